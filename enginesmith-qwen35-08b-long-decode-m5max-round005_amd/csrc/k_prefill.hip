@@ -599,19 +599,39 @@ __global__ __launch_bounds__(256) void k_gdn_prepare_hist(uint16_t* conv, const 
 
 // GDN recurrence over the rows of a chunk (gdn_recur with rows > 1,
 // gdn.metal:176-228), the decode kernel's arithmetic and order per token:
-// block = (16 value rows, head), thread = (row, 8 keys), state in registers
-// for the whole chunk. Tokens go through LDS in tiles of 64, double
-// buffered: the next tile's global loads are issued before the current tile
-// is walked and land in the other buffer after it, one barrier per tile.
-// Within a tile the next token's operands are read from LDS while the
-// current token's chain runs. Lane j of a row keeps the readout of tokens
-// with index j mod 16 and stores them 16 tokens at a time.
-constexpr int kRecurTile = 64;
-struct RecurTileRegs {
-  u32x4 q[4], k[4];
-  uint2 v;
-  float gb;
-};
+// block = (16 value rows, head), four walking waves with thread = (row, 8
+// keys) and the state in registers for the whole chunk, and four staging waves
+// that bring the tokens to LDS as fp32 in tiles of 16, three tiles deep, one
+// barrier per tile.
+//
+// The tokens are a serial chain, so the bound is the walking wave's own
+// instruction stream: per token 8 decays, 8 memory and 8 readout fmas, 8
+// updates, the 4 steps of the memory sum, and 4 LDS reads of k and q. A DPP
+// step that reads a register written by the instruction before it costs two
+// idle issue slots, so the 8 readout fmas of token t - 1 fill those of token
+// t's memory sum (recur_sum_and_readout). The readout needs its own sum
+// across the 16 lanes only once it is stored: 16 tokens' partial sums are
+// reduced together by a transposing tree (33 instructions for 16 tokens
+// instead of 64 plus the selects), which leaves token t's total in one lane.
+// For that tree lane l holds the 8 keys of group recur_group(l), so that the
+// first two of its levels join lanes 8 and 4 apart, where DPP's bank mask
+// selects the token for free; every sum still joins the same key groups in the
+// same order ((0+1)+(2+3))+..., so the bits are the decode kernel's.
+// 4096 tokens: 374 us, 219 cycles a token (570 us with the readout after the
+// update and its own sum per token, and the walking waves staging the tiles).
+// A copy without the LDS reads takes 340 us: the arithmetic's issue is what is
+// left.
+constexpr int kRecurTile = 16;
+// lane of the 16 that hold a row -> key group (8 keys) it holds
+__device__ __forceinline__ int recur_group(int l) {
+  const int hi = (l >> 2) & 1, x = hi ? 3 - (l & 3) : l & 3;
+  return 4 * (((x & 1) << 1) | (x >> 1)) + 2 * hi + (l >> 3);
+}
+// key group -> lane (the inverse)
+__device__ __forceinline__ int recur_lane(int grp) {
+  const int b = grp >> 2, x = ((b & 1) << 1) | (b >> 1);
+  return ((grp & 2) ? 7 - x : x) + 8 * (grp & 1);
+}
 // q, k, v rows are `ld` elements apart (2048 for [m,16,128] arrays, 6144 for
 // the reference's normalised conv buffer [T,6144]); beta is fp32 or, when
 // beta_bf is set, the reference's bf16 [T,16].
@@ -622,138 +642,287 @@ struct RecurIn {
   const float* beta;
   const uint16_t* beta_bf;
 };
-__device__ __forceinline__ void recur_tile_load(const RecurIn& in, int h, int r0, int t0, int nt,
-                                                RecurTileRegs& R) {
-  const int t = threadIdx.x;
-  const int tt = t >> 2, c = (t & 3) * 32;
-  if (tt < nt) {
-    const size_t o = (size_t)(t0 + tt) * in.ld + h * 128 + c;
-    const u32x4* qp = reinterpret_cast<const u32x4*>(in.q + o);
-    const u32x4* kp = reinterpret_cast<const u32x4*>(in.k + o);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      R.q[i] = qp[i];
-      R.k[i] = kp[i];
-    }
-    R.v = *reinterpret_cast<const uint2*>(in.v + (size_t)(t0 + tt) * in.ld + h * 128 + r0 + (t & 3) * 4);
+// LDS tile rows of q and k: 132 floats apart (the tokens a store instruction
+// covers fall in different banks); the keys of lane l's group sit at 4l (first
+// four) and 64 + 4l (last four), so each 16-byte read of a row's 16 lanes
+// covers 256 contiguous bytes. v is kept by row (20 floats apart) and the
+// gates by token, so one 16-byte read fetches four tokens' values.
+constexpr int kRecurRow = 132, kRecurVRow = 20, kRecurRing = 3;
+struct RecurTile {
+  float q[kRecurTile][kRecurRow], k[kRecurTile][kRecurRow];
+  float v[16][kRecurVRow];
+  float g[kRecurTile], beta[kRecurTile];
+};
+// A staging thread's part of a tile: key group t & 15 of q and k of token
+// t >> 4; threads 0..63 four v of token t >> 2; threads 64..95 one gate. Its
+// pointers step a tile at a time; the tokens of a last, partial tile that do
+// not exist repeat the chunk's last token.
+struct RecurStage {
+  const uint16_t *q, *k, *v;
+  size_t gate;  // index into g or beta
+  u32x4 qr, kr;
+  uint2 vr;
+  float gr;
+};
+__device__ __forceinline__ void recur_load(const RecurIn& in, int t, RecurStage& R) {
+  R.qr = *reinterpret_cast<const u32x4*>(R.q);
+  R.kr = *reinterpret_cast<const u32x4*>(R.k);
+  if (t < 64)
+    R.vr = *reinterpret_cast<const uint2*>(R.v);
+  else if (t < 96)
+    R.gr = t < 80 ? in.g[R.gate] : in.beta_bf ? bf2f(in.beta_bf[R.gate]) : in.beta[R.gate];
+}
+// moves R from tile i to tile i + 1 of m tokens
+__device__ __forceinline__ void recur_next(const RecurIn& in, int i, int m, int t, RecurStage& R) {
+  const int first = (i + 1) * kRecurTile, last = m - 1;
+  int dq = kRecurTile, dv = kRecurTile, dg = kRecurTile;
+  if (first + kRecurTile > m) {  // steps that end at the last token
+    dq = min(first + (t >> 4), last) - (i * kRecurTile + (t >> 4));
+    dv = min(first + ((t >> 2) & 15), last) - (i * kRecurTile + ((t >> 2) & 15));
+    dg = min(first + (t & 15), last) - (i * kRecurTile + (t & 15));
   }
-  if (t < 2 * kRecurTile && (t & 63) < nt) {
-    const size_t gi = (size_t)(t0 + (t & 63)) * 16 + h;
-    R.gb = t < 64 ? in.g[gi] : in.beta_bf ? bf2f(in.beta_bf[gi]) : in.beta[gi];
+  R.q += (ptrdiff_t)dq * in.ld;
+  R.k += (ptrdiff_t)dq * in.ld;
+  R.v += (ptrdiff_t)dv * in.ld;
+  R.gate += (ptrdiff_t)dg * 16;
+}
+__device__ __forceinline__ void recur_store(const RecurStage& R, int t, RecurTile& T) {
+  const int l = recur_lane(t & 15);
+  float *qd = &T.q[t >> 4][4 * l], *kd = &T.k[t >> 4][4 * l];
+  *reinterpret_cast<float4*>(qd) = make_float4(bf_lo(R.qr[0]), bf_hi(R.qr[0]), bf_lo(R.qr[1]), bf_hi(R.qr[1]));
+  *reinterpret_cast<float4*>(qd + 64) = make_float4(bf_lo(R.qr[2]), bf_hi(R.qr[2]), bf_lo(R.qr[3]), bf_hi(R.qr[3]));
+  *reinterpret_cast<float4*>(kd) = make_float4(bf_lo(R.kr[0]), bf_hi(R.kr[0]), bf_lo(R.kr[1]), bf_hi(R.kr[1]));
+  *reinterpret_cast<float4*>(kd + 64) = make_float4(bf_lo(R.kr[2]), bf_hi(R.kr[2]), bf_lo(R.kr[3]), bf_hi(R.kr[3]));
+  if (t < 64) {
+    const int tt = t >> 2, rr = (t & 3) * 4;
+    T.v[rr][tt] = bf_lo(R.vr.x);
+    T.v[rr + 1][tt] = bf_hi(R.vr.x);
+    T.v[rr + 2][tt] = bf_lo(R.vr.y);
+    T.v[rr + 3][tt] = bf_hi(R.vr.y);
+  } else if (t < 96) {
+    (t < 80 ? T.g : T.beta)[t & 15] = R.gr;
   }
 }
-// LDS tile rows: 132 floats apart (the 16 rows a store instruction covers
-// fall in different banks); within a row, channel c of 8-channel group j sits
-// at 4j + (c & 3), plus 64 for the group's upper four, so the two 16-byte
-// reads of a row's 16 lanes each cover 256 contiguous bytes.
-constexpr int kRecurRow = 132;
-__device__ __forceinline__ void recur_tile_store(const RecurTileRegs& R, int nt, float (*qs)[kRecurRow],
-                                                 float (*ks)[kRecurRow], float (*vs)[16], float (*gs)[2]) {
-  const int t = threadIdx.x;
-  const int tt = t >> 2, j0 = (t & 3) * 4;
-  if (tt < nt) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int jj = j0 + i;
-      *reinterpret_cast<float4*>(&qs[tt][4 * jj]) =
-          make_float4(bf_lo(R.q[i][0]), bf_hi(R.q[i][0]), bf_lo(R.q[i][1]), bf_hi(R.q[i][1]));
-      *reinterpret_cast<float4*>(&qs[tt][64 + 4 * jj]) =
-          make_float4(bf_lo(R.q[i][2]), bf_hi(R.q[i][2]), bf_lo(R.q[i][3]), bf_hi(R.q[i][3]));
-      *reinterpret_cast<float4*>(&ks[tt][4 * jj]) =
-          make_float4(bf_lo(R.k[i][0]), bf_hi(R.k[i][0]), bf_lo(R.k[i][1]), bf_hi(R.k[i][1]));
-      *reinterpret_cast<float4*>(&ks[tt][64 + 4 * jj]) =
-          make_float4(bf_lo(R.k[i][2]), bf_hi(R.k[i][2]), bf_lo(R.k[i][3]), bf_hi(R.k[i][3]));
-    }
-    const int rr = (t & 3) * 4;
-    vs[tt][rr] = bf_lo(R.v.x);
-    vs[tt][rr + 1] = bf_hi(R.v.x);
-    vs[tt][rr + 2] = bf_lo(R.v.y);
-    vs[tt][rr + 3] = bf_hi(R.v.y);
-  }
-  if (t < 2 * kRecurTile && (t & 63) < nt) gs[t & 63][t >> 6] = R.gb;
+// Sum of mem over the 16 lanes of a row, in all of them (levels: lanes 8
+// apart, the two quads of a half, lanes 2 and 1 apart), with the readout chain
+// o = fma(S[i], q[i], o) from 0 in the slots between its steps: two
+// instructions separate the write of a register from the DPP step that reads
+// it, as the hardware requires.
+__device__ __forceinline__ float recur_sum_and_readout(float& mem, const float (&S)[8], const float (&q)[8]) {
+  float o;
+  asm("v_fma_f32 %1, %2, %10, 0\n\t"
+      "v_fmac_f32 %1, %3, %11\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32 %1, %4, %12\n\t"
+      "v_fmac_f32 %1, %5, %13\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32 %1, %6, %14\n\t"
+      "v_fmac_f32 %1, %7, %15\n\t"
+      "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32 %1, %8, %16\n\t"
+      "v_fmac_f32 %1, %9, %17\n\t"
+      "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+      : "+v"(mem), "=&v"(o)
+      : "v"(S[0]), "v"(S[1]), "v"(S[2]), "v"(S[3]), "v"(S[4]), "v"(S[5]), "v"(S[6]), "v"(S[7]), "v"(q[0]),
+        "v"(q[1]), "v"(q[2]), "v"(q[3]), "v"(q[4]), "v"(q[5]), "v"(q[6]), "v"(q[7]));
+  return o;
 }
-__global__ __launch_bounds__(256, 1) void k_gdn_recur_rows(RecurIn in, int m, float* state, uint16_t* y) {
-  __shared__ __attribute__((aligned(16))) float qs[2][kRecurTile][kRecurRow];
-  __shared__ __attribute__((aligned(16))) float ks[2][kRecurTile][kRecurRow];
-  __shared__ float vs[2][kRecurTile][16];
-  __shared__ float gs[2][kRecurTile][2];
+// The same sum alone.
+__device__ __forceinline__ float recur_sum(float v) {
+  asm("s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+      : "+v"(v));
+  return v;
+}
+// The same sums of 16 tokens' values p: lane l of the row gets the total of
+// token recur_token(l). A level halves the values: the lanes on one side keep
+// the even token of a pair, those on the other side the odd one.
+__device__ __forceinline__ int recur_token(int l) {
+  return (l >> 3) | ((l >> 1) & 2) | ((l << 1) & 4) | ((l & 1) << 3);
+}
+__device__ __forceinline__ float recur_sum16(const float (&p)[16], int l) {
+  float a[8], b[4], c[2];
+  asm("s_nop 1\n\t"
+      "v_add_f32_dpp %0, %8, %8 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %1, %10, %10 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %2, %12, %12 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %3, %14, %14 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %4, %16, %16 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %5, %18, %18 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %6, %20, %20 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %7, %22, %22 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %0, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %1, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %2, %13, %13 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %3, %15, %15 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %4, %17, %17 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %5, %19, %19 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %6, %21, %21 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %7, %23, %23 row_ror:8 row_mask:0xf bank_mask:0xc"
+      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(a[4]), "=&v"(a[5]), "=&v"(a[6]), "=&v"(a[7])
+      : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]), "v"(p[8]),
+        "v"(p[9]), "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
+  asm("s_nop 1\n\t"
+      "v_add_f32_dpp %0, %4, %4 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %1, %6, %6 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %2, %8, %8 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %3, %10, %10 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %0, %5, %5 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %1, %7, %7 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %2, %9, %9 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %3, %11, %11 row_half_mirror row_mask:0xf bank_mask:0xa"
+      : "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]), "=&v"(b[3])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float keep = (l & 2) ? b[2 * i + 1] : b[2 * i], give = (l & 2) ? b[2 * i] : b[2 * i + 1];
+    c[i] = keep + dpp_xor2(give);
+  }
+  const float keep = (l & 1) ? c[1] : c[0], give = (l & 1) ? c[0] : c[1];
+  return keep + dpp_xor1(give);
+}
+__device__ __forceinline__ void recur_read8(const float* row, int l, float (&x)[8]) {
+  const float4 lo = *reinterpret_cast<const float4*>(row + 4 * l), hi = *reinterpret_cast<const float4*>(row + 64 + 4 * l);
+  x[0] = lo.x; x[1] = lo.y; x[2] = lo.z; x[3] = lo.w;
+  x[4] = hi.x; x[5] = hi.y; x[6] = hi.z; x[7] = hi.w;
+}
+__device__ __forceinline__ void recur_read4(const float* p, float (&x)[4]) {
+  const float4 r = *reinterpret_cast<const float4*>(p);
+  x[0] = r.x; x[1] = r.y; x[2] = r.z; x[3] = r.w;
+}
+// The walking wave's operands in flight: k of the token at hand and the next,
+// q of the token before and the one at hand, four tokens' gates and v twice,
+// and the readouts not yet reduced.
+struct RecurWalk {
+  float S[8], k[2][8], q[2][8], g[2][4], be[2][4], v[2][4], p[16];
+};
+// Walks the full tile T; `next` is the tile after it (its first operands are
+// read here). While token u runs, token u + 1's k and token u's q (which the
+// readout uses during token u + 1) are in flight; the fences keep the reads
+// ahead of the arithmetic, and one wait per token covers them all (the
+// compiler's own placement waits three times a token: 389 against 374 us).
+// The tile's own outputs but the last are complete at its end; yprev (when not
+// null) gets the 16 of the tile before.
+__device__ __forceinline__ void recur_walk_tile(const RecurTile& T, const RecurTile& next, int rl, int l, RecurWalk& W,
+                                                uint16_t* yprev) {
+#pragma unroll
+  for (int u = 0; u < kRecurTile; ++u) {
+    const int c = u & 1, f = (u >> 2) & 1;
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads issued a token ago
+    recur_read8(u + 1 < kRecurTile ? T.k[u + 1] : next.k[0], l, W.k[c ^ 1]);
+    if ((u & 3) == 0) {
+      const RecurTile& from = u + 4 < kRecurTile ? T : next;
+      const int u4 = (u + 4) % kRecurTile;
+      recur_read4(&from.g[u4], W.g[f ^ 1]);
+      recur_read4(&from.v[rl][u4], W.v[f ^ 1]);
+      recur_read4(&from.beta[u4], W.be[f ^ 1]);
+    }
+    recur_read8(T.q[u], l, W.q[c]);
+    __builtin_amdgcn_sched_barrier(0);
+    float D[8], mem = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      D[i] = W.S[i] * W.g[f][u & 3];
+      mem = fmaf(D[i], W.k[c][i], mem);
+    }
+    W.p[(u + 15) & 15] = recur_sum_and_readout(mem, W.S, W.q[c ^ 1]);
+    const float delta = (W.v[f][u & 3] - mem) * W.be[f][u & 3];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) W.S[i] = fmaf(W.k[c][i], delta, D[i]);
+    if (u == 0 && yprev) yprev[(size_t)recur_token(l) * 2048] = (uint16_t)f2bf(recur_sum16(W.p, l));
+  }
+}
+__global__ __launch_bounds__(512, 1) void k_gdn_recur_rows(RecurIn in, int m, float* state, uint16_t* y) {
+  __shared__ __attribute__((aligned(16))) RecurTile tile[kRecurRing];
   // blockIdx.x = head, blockIdx.y = block of 16 value rows: the dispatcher
   // deals consecutive blocks to the 8 XCDs in turn, so the 8 row blocks of a
   // head land on one XCD and share its L2 copy of the head's q and k
-  const int t = threadIdx.x, h = blockIdx.x, r0 = blockIdx.y * 16;
-  const int rl = t >> 4, row = r0 + rl, j = t & 15;
-  float* sp = state + ((size_t)(h * 128 + row)) * 128 + 8 * j;
-  const float4 s_lo = reinterpret_cast<const float4*>(sp)[0];
-  const float4 s_hi = reinterpret_cast<const float4*>(sp)[1];
-  float S[8] = {s_lo.x, s_lo.y, s_lo.z, s_lo.w, s_hi.x, s_hi.y, s_hi.z, s_hi.w};
-  RecurTileRegs R;
-  recur_tile_load(in, h, r0, 0, min(kRecurTile, m), R);
-  recur_tile_store(R, min(kRecurTile, m), qs[0], ks[0], vs[0], gs[0]);
-  __syncthreads();
-  uint16_t* yrow = y + h * 128 + row;
-  for (int t0 = 0, buf = 0; t0 < m; t0 += kRecurTile, buf ^= 1) {
-    const int nt = min(kRecurTile, m - t0);
-    const int nt_next = min(kRecurTile, m - t0 - kRecurTile);
-    if (nt_next > 0) recur_tile_load(in, h, r0, t0 + kRecurTile, nt_next, R);
-    // one token: lane j of the row keeps the readout of token index j
-    // within its group of 16; its operands are read one token ahead
-    struct TokOps {
-      float4 k0, k1, q0, q1;
-      float2 gb;
-      float v;
-    };
-    auto operands = [&](int tt) {
-      TokOps o;
-      o.k0 = *reinterpret_cast<const float4*>(&ks[buf][tt][4 * j]);
-      o.k1 = *reinterpret_cast<const float4*>(&ks[buf][tt][64 + 4 * j]);
-      o.q0 = *reinterpret_cast<const float4*>(&qs[buf][tt][4 * j]);
-      o.q1 = *reinterpret_cast<const float4*>(&qs[buf][tt][64 + 4 * j]);
-      o.gb = *reinterpret_cast<const float2*>(&gs[buf][tt][0]);
-      o.v = vs[buf][tt][rl];
-      return o;
-    };
-    auto token = [&](const TokOps& o, int u, float& keep) {
-      const float kk[8] = {o.k0.x, o.k0.y, o.k0.z, o.k0.w, o.k1.x, o.k1.y, o.k1.z, o.k1.w};
-      const float qq[8] = {o.q0.x, o.q0.y, o.q0.z, o.q0.w, o.q1.x, o.q1.y, o.q1.z, o.q1.w};
-      float mem = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        S[i] = S[i] * o.gb.x;
-        mem = fmaf(S[i], kk[i], mem);
+  const int h = blockIdx.x, r0 = blockIdx.y * 16;
+  const int nfull = m / kRecurTile, ntile = (m + kRecurTile - 1) / kRecurTile;
+  // Tile i is walked between barriers i and i + 1, while the staging waves
+  // store tile i + 2 where tile i - 1 was and load tile i + 3; tile i + 1 is
+  // complete, so its first operands are read ahead.
+  if (threadIdx.x >= 256) {  // staging waves
+    const int t = threadIdx.x - 256;
+    RecurStage R;
+    const size_t row = (size_t)min(t >> 4, m - 1) * in.ld + h * 128;
+    R.q = in.q + row + (t & 15) * 8;
+    R.k = in.k + row + (t & 15) * 8;
+    R.v = in.v + (size_t)min((t >> 2) & 15, m - 1) * in.ld + h * 128 + r0 + (t & 3) * 4;
+    R.gate = (size_t)min(t & 15, m - 1) * 16 + h;
+    recur_load(in, t, R);
+    int slot = 0;
+    for (int i = 0; i < ntile; ++i) {  // tile i
+      recur_store(R, t, tile[slot]);
+      slot = slot == kRecurRing - 1 ? 0 : slot + 1;
+      if (i + 1 < ntile) {
+        recur_next(in, i, m, t, R);
+        recur_load(in, t, R);
       }
-      mem = tree16(mem);
-      const float delta = (o.v - mem) * o.gb.y;
-      float out = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        S[i] = fmaf(kk[i], delta, S[i]);
-        out = fmaf(S[i], qq[i], out);
-      }
-      out = tree16(out);
-      keep = u == j ? out : keep;
-    };
-    for (int g0 = 0; g0 < nt; g0 += 16) {
-      const int n16 = min(16, nt - g0);
-      float keep = 0.0f;
-      if (n16 == 16) {
-        TokOps cur = operands(g0);
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-          TokOps nxt;
-          if (u + 1 < 16) nxt = operands(g0 + u + 1);
-          token(cur, u, keep);
-          cur = nxt;
-        }
-      } else {
-        for (int u = 0; u < n16; ++u) token(operands(g0 + u), u, keep);
-      }
-      if (j < n16) yrow[(size_t)(t0 + g0 + j) * 2048] = (uint16_t)f2bf(keep);
+      if (i > 0) __syncthreads();  // barrier i - 1
     }
-    if (nt_next > 0) recur_tile_store(R, nt_next, qs[buf ^ 1], ks[buf ^ 1], vs[buf ^ 1], gs[buf ^ 1]);
-    __syncthreads();
+    __syncthreads();  // barrier ntile - 1
+    __syncthreads();  // barrier ntile
+    return;
   }
-  reinterpret_cast<float4*>(sp)[0] = make_float4(S[0], S[1], S[2], S[3]);
-  reinterpret_cast<float4*>(sp)[1] = make_float4(S[4], S[5], S[6], S[7]);
+  const int t = threadIdx.x, rl = t >> 4, row = r0 + rl, l = t & 15;
+  float* sp = state + ((size_t)(h * 128 + row)) * 128 + 8 * recur_group(l);
+  RecurWalk W;
+  recur_read4(sp, *reinterpret_cast<float(*)[4]>(&W.S[0]));
+  recur_read4(sp + 4, *reinterpret_cast<float(*)[4]>(&W.S[4]));
+#pragma unroll
+  for (int i = 0; i < 8; ++i) W.q[1][i] = 0.0f;
+  uint16_t* yrow = y + h * 128 + row;
+  __syncthreads();  // barrier 0
+  int cur = 0;
+  if (nfull > 0) {
+    recur_read8(tile[0].k[0], l, W.k[0]);
+    recur_read4(&tile[0].g[0], W.g[0]);
+    recur_read4(&tile[0].v[rl][0], W.v[0]);
+    recur_read4(&tile[0].beta[0], W.be[0]);
+    for (int i = 0; i < nfull; ++i) {
+      const int nxt = cur == kRecurRing - 1 ? 0 : cur + 1;
+      recur_walk_tile(tile[cur], tile[nxt], rl, l, W, i > 0 ? yrow + (size_t)(i - 1) * kRecurTile * 2048 : nullptr);
+      cur = nxt;
+      __syncthreads();  // barrier i + 1
+    }
+    float o = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o = fmaf(W.S[i], W.q[1][i], o);
+    W.p[15] = o;
+    yrow[(size_t)((nfull - 1) * kRecurTile + recur_token(l)) * 2048] = (uint16_t)f2bf(recur_sum16(W.p, l));
+  }
+  if (nfull < ntile) {  // the last m % 16 tokens
+    const RecurTile& T = tile[cur];
+    for (int u = 0; u < m - nfull * kRecurTile; ++u) {
+      float k[8], q[8], mem = 0.0f, out = 0.0f;
+      recur_read8(T.k[u], l, k);
+      recur_read8(T.q[u], l, q);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        W.S[i] = W.S[i] * T.g[u];
+        mem = fmaf(W.S[i], k[i], mem);
+      }
+      const float delta = (T.v[rl][u] - recur_sum(mem)) * T.beta[u];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        W.S[i] = fmaf(k[i], delta, W.S[i]);
+        out = fmaf(W.S[i], q[i], out);
+      }
+      out = recur_sum(out);
+      if (l == 0) yrow[(size_t)(nfull * kRecurTile + u) * 2048] = (uint16_t)f2bf(out);
+    }
+    __syncthreads();  // barrier ntile
+  }
+  reinterpret_cast<float4*>(sp)[0] = make_float4(W.S[0], W.S[1], W.S[2], W.S[3]);
+  reinterpret_cast<float4*>(sp)[1] = make_float4(W.S[4], W.S[5], W.S[6], W.S[7]);
 }
 
 // GDN gated norm rows (gdn_norm_gate, gdn.metal:230-255, the decode kernels'
@@ -1226,7 +1395,7 @@ hipError_t launch_gdn_recur_rows(const uint16_t* q, const uint16_t* k, const uin
                                  const float* beta, int m, float* state, uint16_t* y, hipStream_t s) {
   if (!q || !k || !v || !g || !beta || !state || !y || m < 1) return hipErrorInvalidValue;
   const RecurIn in{q, k, v, 2048, g, beta, nullptr};
-  hipLaunchKernelGGL(k_gdn_recur_rows, dim3(kGdnHeads, 8), dim3(256), 0, s, in, m, state, y);
+  hipLaunchKernelGGL(k_gdn_recur_rows, dim3(kGdnHeads, 8), dim3(512), 0, s, in, m, state, y);
   return hipGetLastError();
 }
 
@@ -1258,7 +1427,7 @@ hipError_t launch_gdn_recur_conv(const uint16_t* conv, const float* g, const uin
                                  float* state, uint16_t* y, hipStream_t s) {
   if (!conv || !g || !beta || !state || !y || rows < 1) return hipErrorInvalidValue;
   const RecurIn in{conv, conv + 2048, conv + 4096, kConv, g, nullptr, beta};
-  hipLaunchKernelGGL(k_gdn_recur_rows, dim3(kGdnHeads, 8), dim3(256), 0, s, in, rows, state, y);
+  hipLaunchKernelGGL(k_gdn_recur_rows, dim3(kGdnHeads, 8), dim3(512), 0, s, in, rows, state, y);
   return hipGetLastError();
 }
 

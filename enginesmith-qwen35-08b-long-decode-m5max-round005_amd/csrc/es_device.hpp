@@ -110,11 +110,17 @@ __device__ __forceinline__ void es_sincos(float x, float* sn, float* cs) {
 }
 
 // MLX unary sigmoid in bf16: round after exp, add, reciprocal, subtraction
-// (linear.metal:389-395, gdn.metal:10-15).
+// (linear.metal:389-395, gdn.metal:10-15). The reciprocal is the hardware's
+// (one instruction, within 1 ulp) instead of the correctly rounded division
+// (about ten): d has 8 significant bits and a bf16 rounding boundary of 1/d 9,
+// so 1/d lies at least 2^-17 (relative) away from every boundary and both
+// round to the same bf16. The powers of two keep the reciprocal of a d above
+// 2^126 out of the denormal range, where the instruction returns 0. The input
+// is a bf16 value, so a test compares all 65536.
 __device__ __forceinline__ float sigmoid_bf(float x) {
   const float e = rbf(es_exp(fabsf(x)));
   const float d = rbf(1.0f + e);
-  const float p = rbf(1.0f / d);
+  const float p = rbf(__builtin_amdgcn_rcpf(d * 0.25f) * 0.25f);
   return rbf(x < 0.0f ? p : 1.0f - p);
 }
 

@@ -226,6 +226,9 @@ struct WideGemmArgs {
   int nseg;
   const uint16_t* x;
   int m;
+  // k_q4_gemm, set by its launcher: row tiles dealt to the XCDs; outputs and
+  // residual take 16-byte accesses (aligned, every segment a multiple of 8 wide)
+  int by_xcd, vec;
 };
 hipError_t launch_q4_gemm_stacked(const Q4* w, uint16_t* const* y, int nseg, const uint16_t* x, int m,
                                   hipStream_t s);

@@ -4,16 +4,14 @@
 // k_q4_gemm: Y[M,N] = bf16(X[M,K] . dequant(W)[N,K]^T), optionally
 //   Y = bf16(R + that), as qmm_q4_nax (linear_nax.metal:1096-1139) computes
 //   it: each weight is dequantised to bf16, bf16(scale*q + bias), and the
-//   products accumulate in fp32 (MFMA). Block = 128 rows x 128 features,
-//   four waves of 64 x 64, each a 2 x 2 grid of v_mfma_f32_32x32x16_bf16
-//   tiles. Per 64-wide K step (one quantisation group) the block stages the
-//   X tile and the dequantised W tile in LDS (row stride 72 bf16, so the
-//   16-byte fragment reads of 32 rows spread over the banks), double
-//   buffered: the next step's global loads are in flight while the current
-//   step multiplies.
+//   products accumulate in fp32 (v_mfma_f32_32x32x16_bf16 over K in increasing
+//   order, one chain per output whatever the tiling, so every kernel and tile
+//   height gives the same bits).
 //   Operand layouts (32x32x16 bf16): lane l holds A[l%32][8(l/32)..+7] and
 //   B[8(l/32)..+7][l%32]; result element r of lane l is
 //   D[8(r/4) + 4(l/32) + r%4][l%32].
+#include <type_traits>
+
 #include "es_kernels.hpp"
 
 namespace es {
@@ -28,14 +26,6 @@ template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
-
-constexpr int kGemmBM = 128, kGemmBN = 128, kGemmBK = 64, kGemmLds = 72;
-
-struct GemmStage {
-  u32x4 x[4];    // this thread's 64 bytes of the X tile
-  u32x4 c;       // 32 nibbles of one W row
-  uint32_t s, b; // that row's scale and bias (bf16)
-};
 
 // Two values -> packed bf16 pair (lo in bits 0..15), one v_cvt_pk_bf16_f32.
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) { return pack_bf2(lo, hi); }
@@ -60,128 +50,313 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t word, float sc, float bi) {
   return u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])};
 }
 
-// GATEUP: w is the gate matrix and w2 the up matrix of the MLP; the block's
-// 128 staged W rows are gate rows n0 + 0..31, up rows n0 + 0..31, gate rows
-// n0 + 32..63, up rows n0 + 32..63, so each wave holds a gate and an up
-// accumulator for the same 32 columns and writes
-// act = bf16(bf16(g * sigmoid_bf(g)) * u) with g, u the bf16-rounded GEMM
-// outputs (swiglu_bf16 after the two linears), y [m, N] with N = w.n.
-template <bool GATEUP>
-__global__ __launch_bounds__(256) void k_q4_gemm(Q4 w, Q4 w2, const uint16_t* __restrict__ x, int m,
-                                                 const uint16_t* residual, uint16_t* y) {
-  __shared__ __attribute__((aligned(16))) uint16_t xs[2][kGemmBM][kGemmLds];
-  __shared__ __attribute__((aligned(16))) uint16_t ws[2][kGemmBN][kGemmLds];
+// ---- GEMM: 32 MT x 128 block tiles, weights dequantised in registers ----
+//
+// Block = four waves side by side along N, each 32 MT rows x 32 columns. A
+// lane's 8 values of an MFMA's weight operand are the 8 nibbles of one code
+// word, so a wave dequantises its own columns straight into the operand: no
+// dequantised weight goes through LDS or is made twice in a block. The weights
+// are the MFMA's A operand, so a lane's results are one row and groups of four
+// consecutive columns. X goes through LDS (the four waves read all of it), 64
+// columns of K a step, two stages, one barrier a step; global loads run four
+// steps ahead in registers.
+//
+// A step's arithmetic is 4 MT MFMAs (32 cycles each) and about 115 vector
+// instructions of dequantisation (4 cycles each) that issue in their shadow:
+// MT = 4 balances them, smaller MT repeat the dequantisation for fewer rows.
+// Measured against a 128 x 128 kernel that staged both operands one step ahead
+// and stored its results one by one (us; the third and the last on 256 x 256
+// tiles before):
+//   rows x N x K  203 x 1024 x 3584  4096 x 1024 x 3584  1000 x 4096 x 1024  4096 gate/up  4096 x 6144 x 1024
+//   before              55.7               82                  39                98              82
+//   now                 25.4               44                  16                81              67
+constexpr int kGemmBK = 64, kGemmAhead = 4;
+
+// 16-byte chunk c of 64-column row r: chunk slot c ^ ((r >> 1) & 7), so the 16
+// rows that one 16-lane group of a fragment read touches cover all banks once.
+__device__ __forceinline__ int tile_slot(int r, int c) { return ((c ^ ((r >> 1) & 7)) << 3) + (r << 6); }
+
+// Barrier for LDS data alone: unlike __syncthreads it does not wait for global
+// loads still in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// The code word of slice kk (16 columns of K) for every lane: word 2 kk in
+// lanes 0..31 and word 2 kk + 1 in lanes 32..63.
+__device__ __forceinline__ u32x4 slice_words(const u32x4 c) {
+  const auto p = __builtin_amdgcn_permlane32_swap(c[0], c[1], false, false);  // {w0|w1}, {w4|w5}
+  const auto q = __builtin_amdgcn_permlane32_swap(c[2], c[3], false, false);  // {w2|w3}, {w6|w7}
+  return u32x4{p[0], q[0], p[1], q[1]};
+}
+
+// act = bf16(bf16(g * sigmoid_bf(g)) * u) of the bf16-rounded gate and up
+__device__ __forceinline__ float swiglu(float g, float u) {
+  const float gb = rbf(g), ub = rbf(u);
+  return rbf(rbf(gb * sigmoid_bf(gb)) * ub);
+}
+
+// GATEUP: segment 0 is the gate matrix and segment 1 the up matrix of the MLP;
+// a wave's 32 weight rows are 16 rows of gate and the same 16 of up, so a lane
+// holds both of a column and writes swiglu(g, u) (swiglu_bf16 after the two
+// linears) to y[0] [m, N]. Otherwise the
+// output columns span the stacked segments of a, each written to its own
+// [m][n_s] output; residual (one segment only) may alias y[0].
+//
+// Weights are fetched four steps (256 columns of K, one 128-byte line of codes
+// a row) at a time, eight lanes to a row, and laid down in the wave's own LDS,
+// from which each lane takes its column's words step by step: fetching them a
+// step at a time straight into the lanes that use them touches a line four
+// times, after other rows' lines have evicted it from the L1, and one more line
+// a step for two bytes of scale. LINES: K is a multiple of 256 and the scales
+// allow four-byte accesses; otherwise the loads stay within the row one by one.
+template <int MT, bool GATEUP, bool LINES>
+__global__ __launch_bounds__(256, 2) void k_q4_gemm(WideGemmArgs a, const uint16_t* residual) {
+  constexpr int kRows = 32 * MT, D = kGemmAhead, kCols = GATEUP ? 16 : 32;  // output columns of a wave
+  __shared__ __attribute__((aligned(16))) uint16_t xs[2][kRows * kGemmBK];
+  __shared__ __attribute__((aligned(16))) uint16_t wl[4][32 * kGemmBK];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int n0 = blockIdx.x * (GATEUP ? kGemmBN / 2 : kGemmBN), m0 = blockIdx.y * kGemmBM;
-  const int K = w.k, N = w.n;
-  const int wpr = K >> 3, gpr = K >> 6;
-  // loader roles: X row t/2, 32 columns (t&1); W row t/2, 32 nibbles (t&1)
-  const int lr = t >> 1, lh = t & 1;
-  const Q4& wsrc = (GATEUP && ((lr >> 5) & 1)) ? w2 : w;
-  const int wr = GATEUP ? n0 + (lr >> 6) * 32 + (lr & 31) : n0 + lr;
-  const bool xrow_ok = m0 + lr < m, wrow_ok = wr < N;
-  const uint16_t* xrow = x + (size_t)(xrow_ok ? m0 + lr : 0) * K + lh * 32;
-  const uint32_t* wrow = wsrc.w + (size_t)(wrow_ok ? wr : 0) * wpr + lh * 4;
-  const uint16_t* srow = wsrc.s + (size_t)(wrow_ok ? wr : 0) * gpr;
-  const uint16_t* brow = wsrc.b + (size_t)(wrow_ok ? wr : 0) * gpr;
+  const int fr = lane & 31, fh = lane >> 5;
+  const int K = a.w[0].k, m = a.m, nk = K / kGemmBK;
+  const int ncols = GATEUP ? a.w[0].n : a.nstart[a.nseg];
+  int bx = blockIdx.x, by = blockIdx.y;
+  if (a.by_xcd) {  // block b goes to XCD b % 8: a row tile's blocks share an XCD and its L2's copy of X
+    const int nb = (ncols + 4 * kCols - 1) / (4 * kCols), i = bx >> 3;
+    by = (bx & 7) + 8 * (i / nb);
+    bx = i % nb;
+  }
+  const int m0 = by * kRows;
+  if (m0 >= m) return;
 
-  auto load = [&](int kb, GemmStage& g) {
-    const u32x4* xp = reinterpret_cast<const u32x4*>(xrow + kb * kGemmBK);
+  // Weight rows: lane l fetches chunk l % 8 of rows 8 i + l / 8 (i = 0..3) of
+  // its wave's 32, and the scales (lanes 0..31) or biases (32..63) of row
+  // l % 32. Rows past the end read row 0 and are not stored.
+  const int wn0 = (bx * 4 + wave) * kCols;
+  auto locate = [&](int n, int& seg) {  // n of the wave's 32 -> segment and row in it
+    const int c = wn0 + (GATEUP ? n & 15 : n);
+    seg = GATEUP ? n >> 4 : 0;
+    if (GATEUP) return c < ncols ? c : 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) g.x[i] = xrow_ok ? xp[i] : u32x4{0u, 0u, 0u, 0u};
-    g.c = *reinterpret_cast<const u32x4*>(wrow + kb * 8);
-    g.s = srow[kb];
-    g.b = brow[kb];
+    for (int q = 1; q < 4; ++q)
+      if (q < a.nseg && c < ncols && c >= a.nstart[q]) seg = q;
+    return c < ncols ? c - a.nstart[seg] : 0;
   };
-  auto store = [&](int buf, const GemmStage& g) {
-    u32x4* xd = reinterpret_cast<u32x4*>(&xs[buf][lr][lh * 32]);
+  const uint32_t* cptr[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) xd[i] = g.x[i];
-    // dequantise 32 weights to bf16: bf16(fma(scale, q, bias)); rows past N are 0
-    const float sc = wrow_ok ? bf2f(g.s) : 0.0f, bi = wrow_ok ? bf2f(g.b) : 0.0f;
-    u32x4 o[4];
+  for (int i = 0; i < 4; ++i) {
+    int seg;
+    const int row = locate(8 * i + (lane >> 3), seg);
+    const uint32_t* w = seg == 0 ? a.w[0].w : seg == 1 ? a.w[1].w : seg == 2 ? a.w[2].w : a.w[3].w;
+    cptr[i] = w + (size_t)row * (K >> 3) + (LINES ? (lane & 7) * 4 : 0);
+  }
+  const uint16_t* sptr;
+  {
+    int seg;
+    const int row = locate(fr, seg);
+    const uint16_t* w = fh ? (seg == 0 ? a.w[0].b : seg == 1 ? a.w[1].b : seg == 2 ? a.w[2].b : a.w[3].b)
+                           : (seg == 0 ? a.w[0].s : seg == 1 ? a.w[1].s : seg == 2 ? a.w[2].s : a.w[3].s);
+    sptr = w + (size_t)row * (K >> 6);
+  }
+  // four steps' weights in flight, and the scales and biases of the four at hand
+  u32x4 cq[4];
+  uint2 sq;
+  uint32_t sc4[2], bi4[2];
+  auto load_w = [&](int grp) {
+    // LINES: whole groups only; otherwise a chunk past the row's end repeats its last one
 #pragma unroll
-    for (int wd = 0; wd < 4; ++wd) {
-      o[wd] = dequant8(g.c[wd], sc, bi);
+    for (int i = 0; i < 4; ++i)
+      cq[i] = *reinterpret_cast<const u32x4*>(cptr[i] + (LINES ? grp * 32 : min(grp * 8 + (lane & 7), 2 * nk - 1) * 4));
+    if (LINES) {
+      sq = *reinterpret_cast<const uint2*>(sptr + grp * 4);
+    } else {
+      uint32_t v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = sptr[min(grp * 4 + i, nk - 1)];
+      sq = make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16);
     }
-    u32x4* wd4 = reinterpret_cast<u32x4*>(&ws[buf][lr][lh * 32]);
+  };
+  // the fetched four steps become the ones at hand
+  auto turn_w = [&]() {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) wd4[i] = o[i];
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<u32x4*>(&wl[wave][tile_slot(8 * i + (lane >> 3), lane & 7)]) = cq[i];
+    const auto p = __builtin_amdgcn_permlane32_swap(sq.x, sq.x, false, false);  // {scales|scales}, {biases|biases}
+    const auto q = __builtin_amdgcn_permlane32_swap(sq.y, sq.y, false, false);
+    sc4[0] = p[0]; bi4[0] = p[1];
+    sc4[1] = q[0]; bi4[1] = q[1];
+  };
+  // the lane's words, scale and bias of step u of the four
+  auto words = [&](int u) { return slice_words(*reinterpret_cast<const u32x4*>(&wl[wave][tile_slot(fr, 2 * u + fh)])); };
+  auto scale = [&](int u) { return (u & 1) ? bf_hi(sc4[u >> 1]) : bf_lo(sc4[u >> 1]); };
+  auto bias = [&](int u) { return (u & 1) ? bf_hi(bi4[u >> 1]) : bf_lo(bi4[u >> 1]); };
+
+  // X: thread t moves chunk t & 7 of rows t / 8 + 32 i
+  const int xc = t & 7, xr = t >> 3;
+  const uint16_t* xbase = a.x + (size_t)m0 * K;
+  uint32_t xoff[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) xoff[i] = (uint32_t)min(xr + 32 * i, m - 1 - m0) * (uint32_t)K + xc * 8;
+  auto load_x = [&](int kb, u32x4 (&r)[MT]) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) r[i] = *reinterpret_cast<const u32x4*>((xbase + kb * kGemmBK) + xoff[i]);
+  };
+  auto store_x = [&](int buf, const u32x4 (&r)[MT]) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) *reinterpret_cast<u32x4*>(&xs[buf][tile_slot(xr + 32 * i, xc)]) = r[i];
   };
 
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  const int fr = lane & 31, fk = (lane >> 5) * 8;
-  f32x16 acc[2][2];
+  f32x16 acc[MT];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
 
-  const int nk = K / kGemmBK;
-  GemmStage g;
-  load(0, g);
-  store(0, g);
-  __syncthreads();
-  for (int kb = 0; kb < nk; ++kb) {
-    const int buf = kb & 1;
-    if (kb + 1 < nk) load(kb + 1, g);
+  // Loads are issued in the loop's order, which its waits count: the fences
+  // keep it.
+  const int ngrp = (nk + 3) / 4;
+  u32x4 xq[D][MT];
+  u32x4 bq[4];  // weight operands of a step's four slices
+  load_w(0);
+  issue_fence();
+  load_x(0, xq[0]);
+  issue_fence();
+  turn_w();
+  issue_fence();
+  load_w(min(1, ngrp - 1));
+  issue_fence();
 #pragma unroll
-    for (int kk = 0; kk < kGemmBK; kk += 16) {
-      bf16x8 a[2], b[2];
+  for (int u = 1; u < D; ++u) {
+    load_x(min(u, nk - 1), xq[u]);
+    issue_fence();
+  }
+  store_x(0, xq[0]);
+  load_x(min(D, nk - 1), xq[0]);
+  issue_fence();
+  {
+    const u32x4 wd = words(0);
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-        a[i] = *reinterpret_cast<const bf16x8*>(&xs[buf][wm + 32 * i + fr][kk + fk]);
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        b[j] = *reinterpret_cast<const bf16x8*>(&ws[buf][wn + 32 * j + fr][kk + fk]);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    for (int kk = 0; kk < 4; ++kk) bq[kk] = dequant8(wd[kk], scale(0), bias(0));
+  }
+  lds_barrier();
+  // Step kb = 4 i + u. No step branches, so every wait counts the loads issued
+  // since its own: the loads past the last step repeat it and the X they would
+  // bring goes to a stage nobody reads.
+  auto step = [&](int kb, auto uc) {
+    constexpr int u = decltype(uc)::value, un = (u + 1) % 4;
+    issue_fence();
+    if (u == 3) {
+      turn_w();
+      issue_fence();
+      load_w(min(kb / 4 + 2, ngrp - 1));
     }
-    if (kb + 1 < nk) store(buf ^ 1, g);
-    __syncthreads();
+    // the next step's X to the other stage, whose readers passed the last barrier
+    store_x((u + 1) & 1, xq[un]);
+    load_x(min(kb + 1 + D, nk - 1), xq[un]);
+    const u32x4 wd = words(un);
+    issue_fence();
+    bf16x8 xf[2][MT];
+    auto read_x = [&](int kk) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        xf[kk & 1][i] = *reinterpret_cast<const bf16x8*>(&xs[u & 1][tile_slot(32 * i + fr, 2 * kk + fh)]);
+    };
+    read_x(0);
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      if (kk + 1 < 4) read_x(kk + 1);
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, bq[kk]), xf[kk & 1][i], acc[i], 0, 0, 0);
+      bq[kk] = dequant8(wd[kk], scale(un), bias(un));  // the same slice of the next step
+    }
+    // Issue order: the next slice's fragment reads, then MFMAs each followed by
+    // its share of the dequantisation, which runs in the MFMA's shadow.
+    __builtin_amdgcn_sched_group_barrier(0x100, MT, 0);
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      if (kk + 1 < 4) __builtin_amdgcn_sched_group_barrier(0x100, MT, 0);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 24 / MT, 0);
+      }
+    }
+    issue_fence();
+    lds_barrier();
+  };
+  int k0 = 0;
+  for (; k0 + 4 <= nk; k0 += 4) {
+    step(k0, std::integral_constant<int, 0>{});
+    step(k0 + 1, std::integral_constant<int, 1>{});
+    step(k0 + 2, std::integral_constant<int, 2>{});
+    step(k0 + 3, std::integral_constant<int, 3>{});
+  }
+  if (!LINES) {
+    if (k0 < nk) step(k0, std::integral_constant<int, 0>{});
+    if (k0 + 1 < nk) step(k0 + 1, std::integral_constant<int, 1>{});
+    if (k0 + 2 < nk) step(k0 + 2, std::integral_constant<int, 2>{});
   }
 
-  if (GATEUP) {
+  // Lane l holds row l % 32 of each row tile and, for g = 0..3, weight rows
+  // 8 g + 4 (l / 32) .. + 3 of the wave's 32.
+  auto column = [&](int n, uint16_t*& y, int& ld) {  // output column n -> its matrix and column there
+    int sg = 0;
+    if (!GATEUP) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int col = n0 + wn / 2 + fr;
-      if (col >= N) continue;
+      for (int q = 1; q < 4; ++q)
+        if (q < a.nseg && n >= a.nstart[q]) sg = q;
+    }
+    y = sg == 0 ? a.y[0] : sg == 1 ? a.y[1] : sg == 2 ? a.y[2] : a.y[3];
+    ld = GATEUP ? ncols : a.nstart[sg + 1] - a.nstart[sg];
+    return n - (GATEUP ? 0 : a.nstart[sg]);
+  };
+  auto value = [&](int i, int r) { return GATEUP ? swiglu(acc[i][r], acc[i][(r + 8) & 15]) : acc[i][r]; };
+  uint16_t* y;
+  int ld;
+  if (a.vec) {  // 8 columns and one 16-byte store a lane: the halves of a pair of groups change lanes
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row >= m) continue;
-        const float gb = rbf(acc[i][0][r]), ub = rbf(acc[i][1][r]);
-        const float silu = rbf(gb * sigmoid_bf(gb));
-        y[(size_t)row * N + col] = (uint16_t)f2bf(silu * ub);
+    for (int p = 0; p < kCols / 16; ++p) {
+      const int n = wn0 + 16 * p + 8 * fh;
+      const int col = column(n, y, ld);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = value(i, 8 * p + e);
+        const auto c01 = __builtin_amdgcn_permlane32_swap(pack2(v[0], v[1]), pack2(v[4], v[5]), false, false);
+        const auto c23 = __builtin_amdgcn_permlane32_swap(pack2(v[2], v[3]), pack2(v[6], v[7]), false, false);
+        const int row = m0 + 32 * i + fr;
+        if (row >= m || n >= ncols) continue;
+        u32x4 o = u32x4{c01[0], c23[0], c01[1], c23[1]};
+        const size_t at = (size_t)row * ld + col;
+        if (residual) {
+          const u32x4 rs = *reinterpret_cast<const u32x4*>(residual + at);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = pack2(bf_lo(rs[e]) + bf_lo(o[e]), bf_hi(rs[e]) + bf_hi(o[e]));
+        }
+        *reinterpret_cast<u32x4*>(y + at) = o;
       }
     }
     return;
   }
-  // epilogue: bf16 output, or bf16(residual + bf16(acc))
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = n0 + wn + 32 * j + fr;
-      if (col >= N) continue;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row >= m) continue;
-        const size_t o = (size_t)row * N + col;
-        float v = rbf(acc[i][j][r]);
-        if (residual) v = bf2f(residual[o]) + v;
-        y[o] = (uint16_t)f2bf(v);
-      }
+    for (int r = 0; r < kCols / 2; ++r) {
+      const int row = m0 + 32 * i + fr, n = wn0 + 8 * (r >> 2) + 4 * fh + (r & 3);
+      if (row >= m || n >= ncols) continue;
+      const int col = column(n, y, ld);
+      const size_t o = (size_t)row * ld + col;
+      float v = rbf(value(i, r));
+      if (residual) v = bf2f(residual[o]) + v;
+      y[o] = (uint16_t)f2bf(v);
     }
 }
 
-// ---- wide GEMM: 256 x 256 block tiles for the linears with N >= 2048 ----
+// ---- wide GEMM: 256 x 256 block tiles for a long K and many tiles (wide_ok) ----
 //
 // k_q4_gemm_wide computes the same products as k_q4_gemm, bit for bit: the
 // same bf16 operands (weights dequantised as bf16(fma(scale, q, bias))) and,
@@ -198,14 +373,9 @@ __global__ __launch_bounds__(256) void k_q4_gemm(Q4 w, Q4 w2, const uint16_t* __
 // that belongs in its slot).
 // Output columns may span up to four weight matrices stacked along N
 // (q|k|v, qkv|z|a|b), each written to its own [m][n_s] output.
-// A block holds a whole CU (128 KB of LDS, all registers), so beside the
-// other prefill stream's recurrence or attention it gets fewer CUs than the
-// 128 x 128 kernel, whose blocks share CUs: in the two-stream prefill it pays
-// for the stacked input linears (one launch for four) but not for gate/up,
-// which keeps k_q4_gemm.
+// A block holds a whole CU (128 KB of LDS, all registers), so nothing covers
+// its start and end: it is the faster kernel for a long K only.
 constexpr int kWideM = 256, kWideN = 256, kWideK = 64;
-
-__device__ __forceinline__ int wide_slot(int r, int c) { return ((c ^ ((r >> 1) & 7)) << 3) + (r << 6); }
 
 // Fragment reads as inline assembly: the compiler treats an LDS read after a
 // DMA into LDS as dependent on it and would wait for every DMA in flight
@@ -231,8 +401,8 @@ __device__ __forceinline__ void wide_wait8(u32x4 (&a)[4], u32x4 (&b)[4]) {
 __device__ __forceinline__ void wide_step(uint32_t xt, uint32_t wt, int xrow, int wrow, f32x16 (&acc)[4][4],
                                           int fh) {
   // byte address of slot c of rows xrow (+32i) and wrow (+32j)
-  auto xaddr = [&](int c) { return xt + (uint32_t)(wide_slot(xrow, c) * 2); };
-  auto waddr = [&](int c) { return wt + (uint32_t)(wide_slot(wrow, c) * 2); };
+  auto xaddr = [&](int c) { return xt + (uint32_t)(tile_slot(xrow, c) * 2); };
+  auto waddr = [&](int c) { return wt + (uint32_t)(tile_slot(wrow, c) * 2); };
   u32x4 fa[2][4], fb[2][4];
   wide_read4(xaddr(fh), fa[0][0], fa[0][1], fa[0][2], fa[0][3]);
   wide_read4(waddr(fh), fb[0][0], fb[0][1], fb[0][2], fb[0][3]);
@@ -254,16 +424,6 @@ __device__ __forceinline__ void wide_step(uint32_t xt, uint32_t wt, int xrow, in
                                                             0, 0);
     if (kk + 1 < 4) wide_wait8(fa[cur ^ 1], fb[cur ^ 1]);
   }
-}
-
-// Barrier for the staged tiles: the caller has waited for its own X DMA
-// (vmcnt); lgkmcnt(0) covers the dequantised weights written by ds_write.
-// Unlike __syncthreads it does not wait for the weight loads still in flight.
-__device__ __forceinline__ void wide_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 }
 
 // The two stages are four separate LDS arrays (not one indexed array), so the
@@ -337,7 +497,7 @@ __global__ __launch_bounds__(256, 1) void k_q4_gemm_wide(WideGemmArgs a) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
       const u32x4 o = dequant8(c < 4 ? r.c0[c] : r.c1[c - 4], sc, bi);
-      asm volatile("ds_write_b128 %0, %1" ::"v"(wt + (uint32_t)(wide_slot(t, c) * 2)), "v"(o));
+      asm volatile("ds_write_b128 %0, %1" ::"v"(wt + (uint32_t)(tile_slot(t, c) * 2)), "v"(o));
     }
   };
   // waits for a weight set with N vector-memory operations issued after it
@@ -378,7 +538,7 @@ __global__ __launch_bounds__(256, 1) void k_q4_gemm_wide(WideGemmArgs a) {
   load_w(1, wb);
   wait_set4(wa);
   store_w(lw0, wa);
-  wide_barrier();
+  lds_barrier();
   auto run_step = [&](int st, uint32_t lx, uint32_t lw, uint16_t* x_next, uint32_t lw_next, WRegs& w_next,
                       WRegs& w_after) {
     issue_x(min(st + 1, nk - 1), x_next);
@@ -388,7 +548,7 @@ __global__ __launch_bounds__(256, 1) void k_q4_gemm_wide(WideGemmArgs a) {
     wait_set12(w_next);
     store_w(lw_next, w_next);
     wait_vmcnt<4>();
-    wide_barrier();
+    lds_barrier();
   };
   for (int kb = 0; kb < nk; kb += 2) {  // K is a multiple of 128: nk even
     run_step(kb, lx0, lw0, g_wide_x1, lw1, wb, wa);
@@ -1294,15 +1454,52 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
 
 }  // namespace
 
-// The wide kernel takes a GEMM whose total N fills at least eight of its
-// 256-column tiles; narrower ones (N = 1024 and below, with the residual add)
-// keep the 128 x 128 tiles, which give 256 or more blocks.
-static bool wide_ok(int n_total, int k) { return n_total >= 8 * kWideN && k % (2 * kWideK) == 0; }
+// The wide kernel takes a GEMM without residual whose 256 x 256 tiles fill the
+// CUs (each block has one to itself) in rounds at least seven eighths full and
+// whose K is long enough for its start and end, which nothing else on the CU
+// covers, not to weigh (rows x N x K, wide against the other kernel, us:
+// 4096 x 4096 x 3584 121 and 134, 4096 x 8192 x 4096 266 and 302, but
+// 4096 x 6144 x 1024 81 and 67, 1000 x 8192 x 4096, half a round, 118 and 82).
+static bool wide_ok(int n, int k, int m) {
+  const long tiles = (long)((n + kWideN - 1) / kWideN) * ((m + kWideM - 1) / kWideM), rounds = (tiles + 255) / 256;
+  return k >= 2048 && k % (2 * kWideK) == 0 && tiles >= 224 * rounds;
+}
 
 static hipError_t launch_wide(const WideGemmArgs& a, hipStream_t s) {
   const dim3 grid((a.nstart[a.nseg] + kWideN - 1) / kWideN, (a.m + kWideM - 1) / kWideM);
   hipLaunchKernelGGL(k_q4_gemm_wide, grid, dim3(256), 0, s, a);
   return hipGetLastError();
+}
+
+template <int MT, bool GATEUP>
+static hipError_t launch_gemm_tiles(WideGemmArgs a, const uint16_t* residual, int nb, hipStream_t s) {
+  const int mb = (a.m + 32 * MT - 1) / (32 * MT);
+  a.by_xcd = mb >= 8;  // fewer row tiles than XCDs: blocks in column order reach them all
+  a.vec = ((uintptr_t)residual & 15) == 0;
+  bool lines = a.w[0].k % 256 == 0;
+  for (int i = 0; i < a.nseg; ++i) {
+    a.vec = a.vec && ((uintptr_t)a.y[i] & 15) == 0 && (a.nstart[i + 1] - a.nstart[i]) % 8 == 0;
+    lines = lines && (((uintptr_t)a.w[i].s | (uintptr_t)a.w[i].b) & 3) == 0;
+  }
+  const dim3 grid = a.by_xcd ? dim3(8 * nb * ((mb + 7) / 8)) : dim3(nb, mb);
+  if (lines)
+    hipLaunchKernelGGL((k_q4_gemm<MT, GATEUP, true>), grid, dim3(256), 0, s, a, residual);
+  else
+    hipLaunchKernelGGL((k_q4_gemm<MT, GATEUP, false>), grid, dim3(256), 0, s, a, residual);
+  return hipGetLastError();
+}
+// The smallest row tile whose blocks fit one to a CU (256): below that the
+// chip has CUs to spare and the time is one block's serial walk over K, which
+// a taller tile lengthens; past it the tallest tile dequantises least.
+template <bool GATEUP>
+static hipError_t launch_gemm(const WideGemmArgs& a, const uint16_t* residual, hipStream_t s) {
+  const int n = GATEUP ? a.w[0].n : a.nstart[a.nseg], cols = GATEUP ? 64 : 128;
+  const int nb = (n + cols - 1) / cols;
+  auto blocks = [&](int rows) { return (long)nb * ((a.m + rows - 1) / rows); };
+  if (!GATEUP && !residual && wide_ok(n, a.w[0].k, a.m)) return launch_wide(a, s);
+  if (blocks(32) <= 256) return launch_gemm_tiles<1, GATEUP>(a, residual, nb, s);
+  if (blocks(64) <= 256) return launch_gemm_tiles<2, GATEUP>(a, residual, nb, s);
+  return launch_gemm_tiles<4, GATEUP>(a, residual, nb, s);
 }
 
 hipError_t launch_q4_gemm_stacked(const Q4* w, uint16_t* const* y, int nseg, const uint16_t* x, int m,
@@ -1328,22 +1525,15 @@ hipError_t launch_q4_gemm_stacked(const Q4* w, uint16_t* const* y, int nseg, con
   a.nseg = nseg;
   a.x = x;
   a.m = m;
-  if (wide_ok(n, w[0].k)) return launch_wide(a, s);
-  for (int i = 0; i < nseg; ++i) {
-    const dim3 grid((w[i].n + kGemmBN - 1) / kGemmBN, (m + kGemmBM - 1) / kGemmBM);
-    hipLaunchKernelGGL(k_q4_gemm<false>, grid, dim3(256), 0, s, w[i], w[i], x, m, nullptr, y[i]);
-  }
-  return hipGetLastError();
+  return launch_gemm<false>(a, nullptr, s);
 }
 
 hipError_t launch_q4_gemm(const Q4& w, const uint16_t* x, int m, const uint16_t* residual, uint16_t* y,
                           hipStream_t s) {
   if (!w.w || !w.s || !w.b || w.n < 1 || w.k < kGemmBK || w.k % kGemmBK != 0 || !x || !y || m < 1)
     return hipErrorInvalidValue;
-  if (!residual && wide_ok(w.n, w.k)) return launch_q4_gemm_stacked(&w, &y, 1, x, m, s);
-  const dim3 grid((w.n + kGemmBN - 1) / kGemmBN, (m + kGemmBM - 1) / kGemmBM);
-  hipLaunchKernelGGL(k_q4_gemm<false>, grid, dim3(256), 0, s, w, w, x, m, residual, y);
-  return hipGetLastError();
+  const WideGemmArgs a{{w, w, w, w}, {y, y, y, y}, {0, w.n, w.n, w.n, w.n}, 1, x, m};
+  return launch_gemm<false>(a, residual, s);
 }
 
 hipError_t launch_q4_gemm_swiglu(const Q4& gate, const Q4& up, const uint16_t* x, int m, uint16_t* act,
@@ -1351,9 +1541,8 @@ hipError_t launch_q4_gemm_swiglu(const Q4& gate, const Q4& up, const uint16_t* x
   if (!gate.w || !gate.s || !gate.b || !up.w || !up.s || !up.b || gate.n != up.n || gate.k != up.k ||
       gate.n < 1 || gate.k < kGemmBK || gate.k % kGemmBK != 0 || !x || !act || m < 1)
     return hipErrorInvalidValue;
-  const dim3 grid((gate.n + kGemmBN / 2 - 1) / (kGemmBN / 2), (m + kGemmBM - 1) / kGemmBM);
-  hipLaunchKernelGGL(k_q4_gemm<true>, grid, dim3(256), 0, s, gate, up, x, m, nullptr, act);
-  return hipGetLastError();
+  const WideGemmArgs a{{gate, up, gate, up}, {act, act, act, act}, {0, gate.n, 2 * gate.n, 2 * gate.n, 2 * gate.n}, 2, x, m};
+  return launch_gemm<true>(a, nullptr, s);
 }
 
 }  // namespace es

@@ -61,6 +61,22 @@ __device__ __forceinline__ float es_exp(float x) {
   p = fmaf(p, r, 1.0f);
   return ldexpf(p, (int)n);
 }
+// The same values without branches, for lanes that differ.
+__device__ __forceinline__ float es_exp_sel(float x) {
+  const float n = rintf(x * 1.44269504088896341f);
+  float r = fmaf(n, -0.693145751953125f, x);
+  r = fmaf(n, -1.42860682030941723212e-6f, r);
+  float p = 1.0f / 5040.0f;
+  p = fmaf(p, r, 1.0f / 720.0f);
+  p = fmaf(p, r, 1.0f / 120.0f);
+  p = fmaf(p, r, 1.0f / 24.0f);
+  p = fmaf(p, r, 1.0f / 6.0f);
+  p = fmaf(p, r, 0.5f);
+  p = fmaf(p, r, 1.0f);
+  p = fmaf(p, r, 1.0f);
+  const float e = ldexpf(p, (int)n);
+  return x > 88.72f ? __builtin_inff() : x > -86.0f ? e : 0.0f;
+}
 
 // log for positive normal x: x = m 2^e with m in [sqrt(1/2), sqrt(2)),
 // log m = 2 atanh(s), s = (m-1)/(m+1), series to s^9.
@@ -118,7 +134,7 @@ __device__ __forceinline__ void es_sincos(float x, float* sn, float* cs) {
 // 2^126 out of the denormal range, where the instruction returns 0. The input
 // is a bf16 value, so a test compares all 65536.
 __device__ __forceinline__ float sigmoid_bf(float x) {
-  const float e = rbf(es_exp(fabsf(x)));
+  const float e = rbf(es_exp_sel(fabsf(x)));
   const float d = rbf(1.0f + e);
   const float p = rbf(__builtin_amdgcn_rcpf(d * 0.25f) * 0.25f);
   return rbf(x < 0.0f ? p : 1.0f - p);

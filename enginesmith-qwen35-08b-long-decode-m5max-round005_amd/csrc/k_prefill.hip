@@ -630,8 +630,11 @@ __global__ __launch_bounds__(256) void k_swiglu_rows(const uint16_t* gate, const
 // inputs are the chunk's raw rows, or the ring for positions before the
 // chunk; SiLU; q and k L2-normalised (sum of squares tree64 over channels
 // 0..63 plus tree64 over 64..127) and scaled (q by 1/128, k by bf16(128^-1/2));
-// lane 0 forms the gates g = exp(-exp(A_log)*softplus(bf16(a+dt))), beta =
+// the gates are g = exp(-exp(A_log)*softplus(bf16(a+dt))), beta =
 // sigmoid_bf(b). Outputs bf16 q, k, v [m,16,128] and fp32 g, beta [m,16].
+// Bound by its arithmetic (24 convolutions and SiLUs a lane): 4096 rows take
+// 46 us (86 us with a branch around every load and exponential, and the norms'
+// reciprocals and the gates computed a row at a time).
 constexpr int kPrepRows = 4;  // rows per wave: their taps span kPrepRows + 3 input rows
 __global__ __launch_bounds__(256) void k_gdn_prep_rows(const uint16_t* raw, const uint16_t* ring,
                                                        const uint16_t* conv_w, const uint16_t* a_proj,
@@ -643,34 +646,53 @@ __global__ __launch_bounds__(256) void k_gdn_prep_rows(const uint16_t* raw, cons
   const int t0 = blockIdx.x * kPrepRows;
   if (t0 >= m) return;
   const int nr = min(kPrepRows, m - t0);
+  // input rows t0-3 .. t0+kPrepRows-1: the chunk's raw rows, or the ring for
+  // positions before the chunk; those past the chunk (its last row here) enter
+  // only outputs that are not stored
+  const uint16_t* rows[kPrepRows + 3];
+#pragma unroll
+  for (int i = 0; i < kPrepRows + 3; ++i) {
+    const int tt = t0 - 3 + i;
+    rows[i] = tt >= 0 ? raw + (size_t)min(tt, m - 1) * kConv : ring + (size_t)((pos0 + tt) & 3) * kConv;
+  }
   float out[3][2][kPrepRows];
 #pragma unroll
   for (int part = 0; part < 3; ++part)
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       const int c = part * 2048 + h * 128 + half * 64 + lane;
-      // input rows t0-3 .. t0+kPrepRows-1: the chunk's raw rows, or the ring
-      // for positions before the chunk; rows past the chunk are not used
       uint32_t x[kPrepRows + 3];
 #pragma unroll
-      for (int i = 0; i < kPrepRows + 3; ++i) {
-        const int tt = t0 - 3 + i;
-        x[i] = tt >= 0 ? (tt < m ? raw[(size_t)tt * kConv + c] : 0u)
-                       : ring[(size_t)((pos0 + tt) & 3) * kConv + c];
-      }
+      for (int i = 0; i < kPrepRows + 3; ++i) x[i] = rows[i][c];
       const uint2 w = *reinterpret_cast<const uint2*>(conv_w + (size_t)c * 4);
 #pragma unroll
       for (int r = 0; r < kPrepRows; ++r) out[part][half][r] = conv4_silu(x + r, w);
     }
+  // Lane 2 r + part takes the square-root reciprocal of row r's q (part 0) or k
+  // (part 1), and lane r row r's gates: once for all rows instead of a row at a
+  // time on a wave whose other lanes idle.
+  float tot = 0.0f;
+#pragma unroll
+  for (int r = 0; r < kPrepRows; ++r)
+#pragma unroll
+    for (int part = 0; part < 2; ++part) {
+      const float s2 = tree64(out[part][0][r] * out[part][0][r]) + tree64(out[part][1][r] * out[part][1][r]);
+      tot = lane == 2 * r + part ? s2 : tot;
+    }
+  const float inv_all = 1.0f / sqrtf(tot / 128.0f + 1.0e-6f / 128.0f);
+  if (lane < nr) {
+    const int t = t0 + lane;
+    const float ax = rbf(bf2f(a_proj[(size_t)t * 16 + h]) + bf2f(dt_bias[h]));
+    g[(size_t)t * 16 + h] = es_exp(-es_exp(a_log[h]) * softplus_bf(ax));
+    beta[(size_t)t * 16 + h] = sigmoid_bf(bf2f(b_proj[(size_t)t * 16 + h]));
+  }
 #pragma unroll
   for (int r = 0; r < kPrepRows; ++r) {
     if (r >= nr) break;
-    const int t = t0 + r;
-    const size_t o = ((size_t)t * 16 + h) * 128;
+    const size_t o = ((size_t)(t0 + r) * 16 + h) * 128;
 #pragma unroll
     for (int part = 0; part < 2; ++part) {
-      const float tot = tree64(out[part][0][r] * out[part][0][r]) + tree64(out[part][1][r] * out[part][1][r]);
-      const float inv = 1.0f / sqrtf(tot / 128.0f + 1.0e-6f / 128.0f);
+      const float inv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(inv_all), 2 * r + part));
       const float scale = part == 0 ? 0.0078125f : rbf(0.08838834764831845f);
       uint16_t* dst = part == 0 ? q : k;
       dst[o + lane] = (uint16_t)f2bf(rbf(out[part][0][r] * inv) * scale);
@@ -678,11 +700,6 @@ __global__ __launch_bounds__(256) void k_gdn_prep_rows(const uint16_t* raw, cons
     }
     v[o + lane] = (uint16_t)f2bf(out[2][0][r]);
     v[o + 64 + lane] = (uint16_t)f2bf(out[2][1][r]);
-    if (lane == 0) {
-      const float ax = rbf(bf2f(a_proj[(size_t)t * 16 + h]) + bf2f(dt_bias[h]));
-      g[(size_t)t * 16 + h] = es_exp(-es_exp(a_log[h]) * softplus_bf(ax));
-      beta[(size_t)t * 16 + h] = sigmoid_bf(bf2f(b_proj[(size_t)t * 16 + h]));
-    }
   }
 }
 

@@ -1202,76 +1202,57 @@ __global__ __launch_bounds__(256) void k_attn_gate_rows(const uint16_t* o, const
 // over the cache (attn_prefill, attention_prefill.metal:2256; model.rs:337-343):
 // o = bf16(softmax(q.K^T / 16) . V), fp32 softmax, MFMA products.
 // Block = (32 queries, KV head), 8 waves, two per SIMD: wave w serves query
-// head 4*kvh + (w & 3) for queries 16(w >> 2) .. +15 of the tile. Per block of
-// 32 keys, S^T = K . Q^T on 16x16x32 MFMAs (two 16-key tiles, K from LDS, the
-// wave's Q fragments in registers): lane l holds 8 scores of query l%16, keys
-// 4g + r and 16 + 4g + r (g = l/16, r = 0..3), so the online-softmax max and
-// sum combine 4 lanes with two row exchanges. The exp'ed scores, rounded to
-// bf16, are directly the B operand of O^T += V^T . P^T, with the MFMA's k index
-// 8g + j standing for key (j < 4 ? 4g + j : 16 + 4g + j - 4). Exponentials are
-// base 2 on scores scaled by log2(e)/16.
+// head 4*kvh + (w & 3) for all 32 queries and keys 16(w >> 2) .. +15 of every
+// block of 32 keys, with a softmax state of its own; the two halves are
+// combined at the end. Every K and V fragment a wave reads from LDS so feeds
+// two products: with 16 queries and all 32 keys to a wave the LDS reads (256 KB
+// a key block, 2048 cycles at 128 bytes a cycle) took twice the products' 1024.
+// 4096 queries over 32768 keys, the whole mixer: 1314 -> 1170 us (the kernel at
+// about 0.97 PFLOP/s).
+// S^T = K . Q^T on 16x16x32 MFMAs (16 keys x two groups of 16 queries, K from
+// LDS, Q fragments in registers); a row swap per score leaves lane l with query
+// l % 32 and keys 8(l / 32) .. +7, so the online-softmax max and sum combine
+// two lanes and the exp'ed scores, rounded to bf16, are directly the B operand
+// of O^T += V^T . P^T on 32x32x16 MFMAs. Exponentials are base 2 on scores
+// scaled by log2(e)/16.
 //
 // K and V blocks reach LDS by DMA (global_load_lds, 16 bytes a lane, no
 // registers), kFaStages blocks deep: block kb + kFaStages - 1 is issued while
 // block kb is computed. One DMA instruction moves one 512-byte row (32
-// lanes); K rows sit 528 bytes apart and V rows 544 bytes apart, strides at
+// lanes); K rows sit 528 bytes apart and V rows 576 bytes apart, strides at
 // which the K reads (16 rows x 4 chunks) and the transposing V reads
-// (ds_read_b64_tr_b16: 16 rows x 32 bytes) spread evenly over the banks. The
-// transposing read gives lane i of each 16-lane group element i of the 4 rows
-// x 16 columns its lanes address: lane l gets V[4 keys][d = 16t + l%16]. It is
-// issued as inline assembly with its own lgkmcnt wait, which keeps the
-// compiler from waiting for every DMA in flight before it.
+// (ds_read_b64_tr_b16: 4 rows x 64 bytes a half-wave) spread evenly over the
+// banks. The transposing read gives lane i of each 16-lane group element i of
+// the 4 rows x 16 columns its lanes address: lane l gets V[4 keys][d = 32t +
+// l%32]. It is issued as inline assembly with its own lgkmcnt wait, which keeps
+// the compiler from waiting for every DMA in flight before it.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-constexpr int kFaQ = 32, kFaStages = 4, kFaKs = 264, kFaVs = 272;
+constexpr int kFaQ = 32, kFaStages = 4, kFaKs = 264, kFaVs = 288;
 constexpr int kFaStageHalves = 32 * kFaKs + 32 * kFaVs;
-// sixteen transposing reads from one base: eight at OFF + 32*i (keys 4g..)
-// and eight at kFaHi + OFF + 32*i (keys 16 + 4g..). At most 15 LDS operations
-// are in flight (the width of lgkmcnt): the last read of the second set is
-// issued once the first eight have landed. Every read completes before the
+// Eight transposing reads from one base: keys 0..3 and 4..7 of the lane's eight
+// for four 32-dim tiles at OFF + 64 t. Every read completes before the
 // statement ends.
-constexpr int kFaHi = 2 * 16 * kFaVs;  // bytes from key row 4g to key row 16 + 4g
+constexpr int kFaHi = 2 * 4 * kFaVs;  // bytes from a key row to the fourth after it
 template <int OFF>
-__device__ __forceinline__ void lds_read_tr16_x16(uint32_t a, uint2 (&ra)[8], uint2 (&rb)[8]) {
-  uint64_t x0, x1, x2, x3, x4, x5, x6, x7, y0, y1, y2, y3, y4, y5, y6, y7;
+__device__ __forceinline__ void lds_read_tr16_x8(uint32_t a, u32x4 (&v)[4]) {
+  uint64_t x0, x1, x2, x3, y0, y1, y2, y3;
   asm volatile(
-      "ds_read_b64_tr_b16 %0, %16 offset:%17\n\t"
-      "ds_read_b64_tr_b16 %1, %16 offset:%17+32\n\t"
-      "ds_read_b64_tr_b16 %2, %16 offset:%17+64\n\t"
-      "ds_read_b64_tr_b16 %3, %16 offset:%17+96\n\t"
-      "ds_read_b64_tr_b16 %4, %16 offset:%17+128\n\t"
-      "ds_read_b64_tr_b16 %5, %16 offset:%17+160\n\t"
-      "ds_read_b64_tr_b16 %6, %16 offset:%17+192\n\t"
-      "ds_read_b64_tr_b16 %7, %16 offset:%17+224\n\t"
-      "ds_read_b64_tr_b16 %8, %16 offset:%18\n\t"
-      "ds_read_b64_tr_b16 %9, %16 offset:%18+32\n\t"
-      "ds_read_b64_tr_b16 %10, %16 offset:%18+64\n\t"
-      "ds_read_b64_tr_b16 %11, %16 offset:%18+96\n\t"
-      "ds_read_b64_tr_b16 %12, %16 offset:%18+128\n\t"
-      "ds_read_b64_tr_b16 %13, %16 offset:%18+160\n\t"
-      "ds_read_b64_tr_b16 %14, %16 offset:%18+192\n\t"
-      "s_waitcnt lgkmcnt(7)\n\t"
-      "ds_read_b64_tr_b16 %15, %16 offset:%18+224\n\t"
+      "ds_read_b64_tr_b16 %0, %8 offset:%9\n\t"
+      "ds_read_b64_tr_b16 %4, %8 offset:%10\n\t"
+      "ds_read_b64_tr_b16 %1, %8 offset:%9+64\n\t"
+      "ds_read_b64_tr_b16 %5, %8 offset:%10+64\n\t"
+      "ds_read_b64_tr_b16 %2, %8 offset:%9+128\n\t"
+      "ds_read_b64_tr_b16 %6, %8 offset:%10+128\n\t"
+      "ds_read_b64_tr_b16 %3, %8 offset:%9+192\n\t"
+      "ds_read_b64_tr_b16 %7, %8 offset:%10+192\n\t"
       "s_waitcnt lgkmcnt(0)"
-      : "=&v"(x0), "=&v"(x1), "=&v"(x2), "=&v"(x3), "=&v"(x4), "=&v"(x5), "=&v"(x6), "=&v"(x7),
-        "=&v"(y0), "=&v"(y1), "=&v"(y2), "=&v"(y3), "=&v"(y4), "=&v"(y5), "=&v"(y6), "=&v"(y7)
+      : "=&v"(x0), "=&v"(x1), "=&v"(x2), "=&v"(x3), "=&v"(y0), "=&v"(y1), "=&v"(y2), "=&v"(y3)
       : "v"(a), "n"(OFF), "n"(kFaHi + OFF)
       : "memory");
-  ra[0] = __builtin_bit_cast(uint2, x0);
-  ra[1] = __builtin_bit_cast(uint2, x1);
-  ra[2] = __builtin_bit_cast(uint2, x2);
-  ra[3] = __builtin_bit_cast(uint2, x3);
-  ra[4] = __builtin_bit_cast(uint2, x4);
-  ra[5] = __builtin_bit_cast(uint2, x5);
-  ra[6] = __builtin_bit_cast(uint2, x6);
-  ra[7] = __builtin_bit_cast(uint2, x7);
-  rb[0] = __builtin_bit_cast(uint2, y0);
-  rb[1] = __builtin_bit_cast(uint2, y1);
-  rb[2] = __builtin_bit_cast(uint2, y2);
-  rb[3] = __builtin_bit_cast(uint2, y3);
-  rb[4] = __builtin_bit_cast(uint2, y4);
-  rb[5] = __builtin_bit_cast(uint2, y5);
-  rb[6] = __builtin_bit_cast(uint2, y6);
-  rb[7] = __builtin_bit_cast(uint2, y7);
+  const uint64_t x[4] = {x0, x1, x2, x3}, y[4] = {y0, y1, y2, y3};
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    v[t] = u32x4{(uint32_t)x[t], (uint32_t)(x[t] >> 32), (uint32_t)y[t], (uint32_t)(y[t] >> 32)};
 }
 // max of two scores by v_max_f32 alone: scores are never NaN, so the operand
 // canonicalisation that fmaxf adds changes nothing and is left out
@@ -1284,30 +1265,35 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
                                                          const uint16_t* vcache, int pos0, int m,
                                                          int capacity, uint16_t* o) {
   __shared__ __attribute__((aligned(16))) uint16_t kv[kFaStages][kFaStageHalves];
+  __shared__ uint32_t merged[4];
+  static_assert(sizeof(kv) >= 4 * (32 * 256 + 128) * sizeof(float), "the merge fits the staging memory");
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // uniform: scalar DMA addressing
+  if (t < 4) merged[t] = 0;
   // 1-D grid dealt to the 8 XCDs in turn (block b on XCD b % 8): XCDs
   // 0, 2, 4, 6 take KV head 0 and 1, 3, 5, 7 head 1, so the query tiles that
   // stream one head's K and V share an XCD's L2
   const int b = blockIdx.x, xcd = b & 7;
   const int tile = 4 * (b >> 3) + (xcd >> 1);
   if (tile * kFaQ >= m) return;
-  const int t0 = tile * kFaQ, kvh = xcd & 1, hq = 4 * kvh + (wave & 3);
+  const int t0 = tile * kFaQ, kvh = xcd & 1, hq = 4 * kvh + (wave & 3), kh = wave >> 2;
   const int qi = lane & 15, g = lane >> 4;
-  const int qrow = t0 + 16 * (wave >> 2) + qi;
+  const int qrow = t0 + (lane & 31);  // the lane's query once the scores are swapped
   const bool qvalid = qrow < m;
   const int qpos = pos0 + (qvalid ? qrow : m - 1);
   const int last_key = pos0 + min(t0 + kFaQ, m) - 1;
   const int nkb = last_key / 32 + 1;
-  // Q fragments: B operand of k-step s holds Q[q][32s + 8g .. +7]
-  bf16x8 qf[8];
-  {
-    const uint16_t* qp = qr + ((size_t)(qvalid ? qrow : 0) * 8 + hq) * 256 + 8 * g;
+  // Q fragments: B operand of k-step s for query group u holds Q[16u + q][32s + 8g .. +7]
+  bf16x8 qf[2][8];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int r = t0 + 16 * u + qi;
+    const uint16_t* qp = qr + ((size_t)(r < m ? r : 0) * 8 + hq) * 256 + 8 * g;
 #pragma unroll
     for (int s2 = 0; s2 < 8; ++s2) {
       u32x4 v = *reinterpret_cast<const u32x4*>(qp + 32 * s2);
-      if (!qvalid) v = u32x4{0u, 0u, 0u, 0u};
-      qf[s2] = __builtin_bit_cast(bf16x8, v);
+      if (r >= m) v = u32x4{0u, 0u, 0u, 0u};
+      qf[u][s2] = __builtin_bit_cast(bf16x8, v);
     }
   }
   // DMA of one block of 32 keys: wave w moves rows 4w .. 4w+3 of K and V,
@@ -1337,20 +1323,23 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
     }
   };
   for (int kb = 0; kb < min(kFaStages - 1, nkb); ++kb) issue(kb);
-  f32x4 ot[16];
+  f32x16 ot[8];  // O^T: dims 32t + 8(r/4) + 4(l/32) + r%4 of query l % 32
 #pragma unroll
-  for (int dt = 0; dt < 16; ++dt)
+  for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ot[dt][r] = 0.0f;
-  float mrun = -INFINITY, lrun = 0.0f;
+    for (int r = 0; r < 16; ++r) ot[dt][r] = 0.0f;
+  // The running reference starts below every score but finite: a row may have
+  // no key in this wave's half of its blocks (or none before them), and
+  // -inf - -inf would be NaN.
+  float mrun = -3.0e38f, lrun = 0.0f;
   const float c = 0.0625f * 1.4426950408889634f;  // 1/16 * log2(e)
-  // V read roles (see above): lane address row K0 + (l%16)/4, columns
-  // 4((l%16)%4) of the first 16-dim tile, K0 = 4g (keys of k indices 0..3)
-  // or 16 + 4g (k indices 4..7)
   const uint32_t kv_base =
       (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) uint16_t*)(&kv[0][0]));
-  const uint32_t v_lane = (uint32_t)(2 * (32 * kFaKs + (4 * g + (qi >> 2)) * kFaVs + 4 * (qi & 3)));
-  for (int kb = 0; kb < nkb; ++kb) {
+  // V reads (see above): 16-lane group g takes dims 16(g & 1) .. of a tile and
+  // keys 8(g / 2) .. of the wave's 16
+  const uint32_t v_lane =
+      (uint32_t)(2 * (32 * kFaKs + (16 * kh + 8 * (g >> 1) + (qi >> 2)) * kFaVs + 16 * (g & 1) + 4 * (qi & 3)));
+  for (int kb = 0;; ++kb) {
     // blocks issued after kb and still in flight: min(kFaStages - 2, nkb-1-kb),
     // 8 DMA instructions each per wave
     const int ahead = min(kFaStages - 2, nkb - 1 - kb);
@@ -1361,20 +1350,17 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
     else
       wait_vmcnt<0>();
     __syncthreads();  // block kb visible; every wave is past block kb-1
-    const uint16_t* ks = kv[kb % kFaStages];
+    if (kb == nkb) break;  // every wave is past the last block: the staging memory is free
+    const uint16_t* ks = kv[kb % kFaStages] + 16 * kh * kFaKs;
     const uint32_t vs_addr = kv_base + (uint32_t)(2 * kFaStageHalves * (kb % kFaStages)) + v_lane;
-    // scores S^T[key][q] for the two 16-key tiles of this block
-    // The K fragments of k-steps s2 .. s2 + 3 are in flight while step s2's
-    // two products run (fences keep the order), so each pair of products
-    // waits for its own reads only.
+    // scores S^T[key][q] for the two groups of 16 queries. The K fragments of
+    // k-steps s2 .. s2 + 3 are in flight while step s2's two products run
+    // (fences keep the order), so each pair of products waits for its own read
+    // only.
     f32x4 st[2];
     {
-      bf16x8 kf[2][8];
-      auto read_k = [&](int s2) {
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-          kf[kt][s2] = *reinterpret_cast<const bf16x8*>(ks + (16 * kt + qi) * kFaKs + 32 * s2 + 8 * g);
-      };
+      bf16x8 kf[8];
+      auto read_k = [&](int s2) { kf[s2] = *reinterpret_cast<const bf16x8*>(ks + qi * kFaKs + 32 * s2 + 8 * g); };
 #pragma unroll
       for (int s2 = 0; s2 < 4; ++s2) read_k(s2);
       // block kb + 3 goes to the stage every wave finished before the barrier;
@@ -1382,38 +1368,40 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
       if (kb + kFaStages - 1 < nkb) issue(kb + kFaStages - 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) st[kt][r] = 0.0f;
+        for (int r = 0; r < 4; ++r) st[u][r] = 0.0f;
 #pragma unroll
       for (int s2 = 0; s2 < 8; ++s2) {
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-          st[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kt][s2], qf[s2], st[kt], 0, 0, 0);
+        for (int u = 0; u < 2; ++u)
+          st[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s2], qf[u][s2], st[u], 0, 0, 0);
         if (s2 + 4 < 8) read_k(s2 + 4);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    // lane l: keys 4g + r of query l % 16 of both groups -> keys 8(l / 32) + e
+    // of query l % 32
     float x[8];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) x[4 * kt + r] = st[kt][r];
+    for (int r = 0; r < 4; ++r) {
+      const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(st[0][r]), __float_as_uint(st[1][r]), false, false);
+      x[r] = __uint_as_float(p[0]);
+      x[4 + r] = __uint_as_float(p[1]);
+    }
     // causal mask (only blocks that reach past the tile's first query),
-    // online softmax for query qi; the maximum is taken on the raw scores
-    // (scaling by c > 0 keeps the order) and the exponent is fma(s, c, -max)
+    // online softmax for the lane's query; the maximum is taken on the raw
+    // scores (scaling by c > 0 keeps the order) and the exponent is
+    // fma(s, c, -max)
     if (kb * 32 + 31 > pos0 + t0) {
+      const int key0 = kb * 32 + 16 * kh + 8 * (lane >> 5);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int key = kb * 32 + 16 * (e >> 2) + 4 * g + (e & 3);
-        x[e] = key <= qpos ? x[e] : -INFINITY;
-      }
+      for (int e = 0; e < 8; ++e) x[e] = key0 + e <= qpos ? x[e] : -INFINITY;
     }
     float mloc = x[0];
 #pragma unroll
     for (int e = 1; e < 8; ++e) mloc = fmaxf(mloc, x[e]);
-    const float2 m16 = rows_xor16(mloc);
-    const float2 m32 = rows_xor32(max_raw(m16.x, m16.y));
+    const float2 m32 = rows_xor32(mloc);
     // The exponent's reference value moves only when the block's maximum
     // exceeds it by more than 8 (probabilities stay below 2^8; the output is
     // normalised by a sum taken against the same reference, so the softmax is
@@ -1429,8 +1417,7 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
     float psum = pv[0];
 #pragma unroll
     for (int e = 1; e < 8; ++e) psum += pv[e];
-    const float2 s16 = rows_xor16(psum);
-    const float2 s32 = rows_xor32(s16.x + s16.y);
+    const float2 s32 = rows_xor32(psum);
     lrun = lrun * factor + (s32.x + s32.y);
     const float mrun_old = mrun;
     mrun = mnew;
@@ -1438,35 +1425,59 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
     // skipped unless some lane's reference moved
     if (__any(mnew > mrun_old)) {
 #pragma unroll
-      for (int dt = 0; dt < 16; ++dt)
+      for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ot[dt][r] *= factor;
+        for (int r = 0; r < 16; ++r) ot[dt][r] *= factor;
     }
-    // O^T += V^T . P^T: one 32-key step per 16-dim tile
+    // O^T += V^T . P^T: one 16-key step per 32-dim tile
     const u32x4 pb = u32x4{pack2(pv[0], pv[1]), pack2(pv[2], pv[3]), pack2(pv[4], pv[5]), pack2(pv[6], pv[7])};
     const bf16x8 pf = __builtin_bit_cast(bf16x8, pb);
 #pragma unroll
-    for (int d8 = 0; d8 < 2; ++d8) {
-      uint2 lo[8], hi[8];
-      if (d8 == 0)
-        lds_read_tr16_x16<0>(vs_addr, lo, hi);
+    for (int d4 = 0; d4 < 2; ++d4) {
+      u32x4 vf[4];
+      if (d4 == 0)
+        lds_read_tr16_x8<0>(vs_addr, vf);
       else
-        lds_read_tr16_x16<256>(vs_addr, lo, hi);
+        lds_read_tr16_x8<256>(vs_addr, vf);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int dt = 8 * d8 + i;
-        const bf16x8 vf = __builtin_bit_cast(bf16x8, u32x4{lo[i].x, lo[i].y, hi[i].x, hi[i].y});
-        ot[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, ot[dt], 0, 0, 0);
-      }
+      for (int i = 0; i < 4; ++i)
+        ot[4 * d4 + i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[i]), pf, ot[4 * d4 + i], 0, 0, 0);
     }
   }
-  if (!qvalid) return;
-  const float inv = 1.0f / lrun;
-  uint16_t* op = o + ((size_t)qrow * 8 + hq) * 256 + 4 * g;
+  // The upper half's wave leaves its state in the staging memory and raises its
+  // flag; the lower half's waits for it (the other wave runs on this CU and
+  // waits for nothing, so the wait ends) and writes the result.
+  float* merge = reinterpret_cast<float*>(&kv[0][0]) + (wave & 3) * (32 * 256 + 128);
+  if (kh) {
 #pragma unroll
-  for (int dt = 0; dt < 16; ++dt)
-    *reinterpret_cast<uint2*>(op + 16 * dt) =
-        make_uint2(pack2(ot[dt][0] * inv, ot[dt][1] * inv), pack2(ot[dt][2] * inv, ot[dt][3] * inv));
+    for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<float4*>(merge + ((4 * dt + r) * 64 + lane) * 4) =
+            make_float4(ot[dt][4 * r], ot[dt][4 * r + 1], ot[dt][4 * r + 2], ot[dt][4 * r + 3]);
+    merge[32 * 256 + lane] = mrun;
+    merge[32 * 256 + 64 + lane] = lrun;
+    __hip_atomic_store(&merged[wave & 3], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    return;
+  }
+  while (__hip_atomic_load(&merged[wave & 3], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
+    __builtin_amdgcn_s_sleep(1);
+  if (!qvalid) return;
+  // Key 0 is in the lower half, so mrun is a score's and the sum is not 0; an
+  // upper half without keys has weight 0.
+  const float m1 = merge[32 * 256 + lane], l1 = merge[32 * 256 + 64 + lane];
+  const float mx = fmaxf(mrun, m1), f0 = __builtin_amdgcn_exp2f(mrun - mx), f1 = __builtin_amdgcn_exp2f(m1 - mx);
+  const float inv = 1.0f / (lrun * f0 + l1 * f1), i0 = f0 * inv, i1 = f1 * inv;
+  uint16_t* op = o + ((size_t)qrow * 8 + hq) * 256 + 4 * (lane >> 5);
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float4 u = *reinterpret_cast<const float4*>(merge + ((4 * dt + r) * 64 + lane) * 4);
+      *reinterpret_cast<uint2*>(op + 32 * dt + 8 * r) =
+          make_uint2(pack2(fmaf(ot[dt][4 * r], i0, u.x * i1), fmaf(ot[dt][4 * r + 1], i0, u.y * i1)),
+                     pack2(fmaf(ot[dt][4 * r + 2], i0, u.z * i1), fmaf(ot[dt][4 * r + 3], i0, u.w * i1)));
+    }
 }
 
 }  // namespace

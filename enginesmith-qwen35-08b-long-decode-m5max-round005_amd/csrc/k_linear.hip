@@ -576,24 +576,49 @@ hipError_t launch_norm_gate_up_parts(const Q4& gate, const Q4& up, const uint16_
   return hipGetLastError();
 }
 
+// A wave unpacks and sums its slices of x once for its P weight rows (about
+// 100 instructions a slice, more than a row's dot product over it). One token
+// row has fewer waves than the chip has SIMDs, so P is small there; several
+// token rows take P = 4 once its waves fill the SIMDs (once for whole-wave
+// rows, twice for half-wave rows, whose P = 2 already holds four). us with the
+// small P and with 4, 11 token rows: 1024 x 3584 8.3 and 6.4, 3584 x 1024 5.65
+// and 5.2; 32 rows: 19.0 and 11.9, 12.2 and 10.0; at the line nothing either
+// way; P = 8 is slower again.
+constexpr int kRowsP = 4;
+constexpr long kSimds = 1024;
+template <int P>
+static void launch_qmv_narrow_p(const Q4& w, const uint16_t* x, int rows, const uint16_t* residual, uint16_t* y,
+                                float* y_f32, hipStream_t s) {
+  const dim3 grid((w.n + 8 * P - 1) / (8 * P), rows);
+  if (residual)
+    hipLaunchKernelGGL((k_qmv_narrow<P, true>), grid, dim3(256), 0, s, w, x, residual, y, y_f32);
+  else
+    hipLaunchKernelGGL((k_qmv_narrow<P, false>), grid, dim3(256), 0, s, w, x, residual, y, y_f32);
+}
+template <int P>
+static void launch_qmv_wide_p(const Q4& w, const uint16_t* x, int rows, const uint16_t* residual, uint16_t* y,
+                              float* y_f32, hipStream_t s) {
+  const dim3 grid((w.n + 4 * P - 1) / (4 * P), rows);
+  if (residual)
+    hipLaunchKernelGGL((k_qmv_wide<P, true>), grid, dim3(256), 0, s, w, x, residual, y, y_f32);
+  else
+    hipLaunchKernelGGL((k_qmv_wide<P, false>), grid, dim3(256), 0, s, w, x, residual, y, y_f32);
+}
+
 hipError_t launch_qmv_rows(const Q4& w, const uint16_t* x, int rows, const uint16_t* residual,
                            uint16_t* y, float* y_f32, hipStream_t s) {
   if (!q4_ok(w) || !x || !y || rows < 1 || rows > 65535 || (y_f32 && rows != 1))
     return hipErrorInvalidValue;
   if (w.k == kHidden) {
-    const int rpb = 4 * 2 * kNarrowP;
-    const dim3 grid((w.n + rpb - 1) / rpb, rows);
-    if (residual)
-      hipLaunchKernelGGL((k_qmv_narrow<kNarrowP, true>), grid, dim3(256), 0, s, w, x, residual, y, y_f32);
+    if (rows > 1 && (long)rows * w.n > 2 * kSimds * 2 * kRowsP)
+      launch_qmv_narrow_p<kRowsP>(w, x, rows, residual, y, y_f32, s);
     else
-      hipLaunchKernelGGL((k_qmv_narrow<kNarrowP, false>), grid, dim3(256), 0, s, w, x, residual, y, y_f32);
+      launch_qmv_narrow_p<kNarrowP>(w, x, rows, residual, y, y_f32, s);
   } else if (w.k > kHidden && w.k <= 4096) {
-    const int rpb = 4 * kWideP;
-    const dim3 grid((w.n + rpb - 1) / rpb, rows);
-    if (residual)
-      hipLaunchKernelGGL((k_qmv_wide<kWideP, true>), grid, dim3(256), 0, s, w, x, residual, y, y_f32);
+    if (rows > 1 && (long)rows * w.n >= kSimds * kRowsP)
+      launch_qmv_wide_p<kRowsP>(w, x, rows, residual, y, y_f32, s);
     else
-      hipLaunchKernelGGL((k_qmv_wide<kWideP, false>), grid, dim3(256), 0, s, w, x, residual, y, y_f32);
+      launch_qmv_wide_p<kWideP>(w, x, rows, residual, y, y_f32, s);
   } else {
     return hipErrorInvalidValue;
   }

@@ -27,3 +27,20 @@ def test_every_bf16_value():
     want, got = O.swiglu(x, one), act.numpy(np.uint16)
     nan = ((want & 0x7FFF) > 0x7F80) & ((got & 0x7FFF) > 0x7F80)  # a NaN's payload is not specified
     assert_bits_equal(np.where(nan, 0, got), np.where(nan, 0, want), what="silu")
+
+
+@pytest.mark.parametrize("off", [0, 1])
+def test_gate_rows_aligned_and_not(off):
+    """Pointers `off` bf16 elements past 16-byte alignment take the element
+    form, aligned ones the 8-element form: the same bits, in place too."""
+    r = np.random.default_rng(7)
+    m = 3
+    o = O.f32_to_bf16(r.normal(0, 1, m * 2048).astype(np.float32))
+    qp = O.f32_to_bf16(r.normal(0, 2, m * 4096).astype(np.float32))
+    pad = np.zeros(off, np.uint16)
+    do, dq = (E.DeviceBuffer.from_numpy(np.concatenate([pad, a])) for a in (o, qp))
+    E.check(E.lib().es_attn_gate_rows(do.ptr + 2 * off, dq.ptr + 2 * off, m, do.ptr + 2 * off, None))
+    E.synchronize()
+    got = do.numpy(np.uint16)[off:].reshape(m, 2048)
+    for t in range(m):
+        assert_bits_equal(got[t], O.attn_gate(o[2048 * t:2048 * t + 2048], qp[4096 * t:4096 * t + 4096]), what=f"row {t}")

@@ -1223,8 +1223,8 @@ __global__ __launch_bounds__(256) void k_attn_gate_rows(const uint16_t* o, const
 // combined at the end. Every K and V fragment a wave reads from LDS so feeds
 // two products: with 16 queries and all 32 keys to a wave the LDS reads (256 KB
 // a key block, 2048 cycles at 128 bytes a cycle) took twice the products' 1024.
-// 4096 queries over 32768 keys, the whole mixer: 1314 -> 1170 us (the kernel at
-// about 0.97 PFLOP/s).
+// 4096 queries over 32768 keys: 1141 -> 1023 us in a graph's replay, 1.0
+// PFLOP/s (1237 us after under the profiler, whose runs clock lower).
 // S^T = K . Q^T on 16x16x32 MFMAs (16 keys x two groups of 16 queries, K from
 // LDS, Q fragments in registers); a row swap per score leaves lane l with query
 // l % 32 and keys 8(l / 32) .. +7, so the online-softmax max and sum combine
@@ -1245,6 +1245,10 @@ __global__ __launch_bounds__(256) void k_attn_gate_rows(const uint16_t* o, const
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kFaQ = 32, kFaStages = 4, kFaKs = 264, kFaVs = 288;
 constexpr int kFaStageHalves = 32 * kFaKs + 32 * kFaVs;
+constexpr int kFaMerge = 64 * 66;  // floats a wave leaves for the other: 64 sums, the reference and the sum a lane
+constexpr int kFaQRow = 136;  // bf16 elements between 128-element Q rows in LDS: spread over the banks as the K rows
+typedef u32x4 __attribute__((aligned(8))) u32x4_a8;
+static_assert(kFaStageHalves >= 8 * 16 * kFaQRow, "the waves' Q rows fit a stage");
 // Eight transposing reads from one base: keys 0..3 and 4..7 of the lane's eight
 // for four 32-dim tiles at OFF + 64 t. Every read completes before the
 // statement ends.
@@ -1281,11 +1285,11 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
                                                          const uint16_t* vcache, int pos0, int m,
                                                          int capacity, uint16_t* o) {
   __shared__ __attribute__((aligned(16))) uint16_t kv[kFaStages][kFaStageHalves];
-  __shared__ uint32_t merged[4];
-  static_assert(sizeof(kv) >= 4 * (32 * 256 + 128) * sizeof(float), "the merge fits the staging memory");
+  __shared__ uint32_t merged[8];
+  static_assert(sizeof(kv) >= 8 * kFaMerge * sizeof(float), "the merge fits the staging memory");
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // uniform: scalar DMA addressing
-  if (t < 4) merged[t] = 0;
+  if (t < 8) merged[t] = 0;
   // 1-D grid dealt to the 8 XCDs in turn (block b on XCD b % 8): XCDs
   // 0, 2, 4, 6 take KV head 0 and 1, 3, 5, 7 head 1, so the query tiles that
   // stream one head's K and V share an XCD's L2
@@ -1299,19 +1303,19 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
   const int qpos = pos0 + (qvalid ? qrow : m - 1);
   const int last_key = pos0 + min(t0 + kFaQ, m) - 1;
   const int nkb = last_key / 32 + 1;
-  // Q fragments: B operand of k-step s for query group u holds Q[16u + q][32s + 8g .. +7]
-  bf16x8 qf[2][8];
+  // Q by whole lines, four rows of 256 bytes an instruction: fetched straight
+  // into the fragments' lanes (64 bytes of 16 rows an instruction) the block's
+  // 128 loads took 8,500 cycles to issue. A query past m reads the last one; its
+  // results are not stored.
+  u32x4 qv[2][2][4];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int r = t0 + 16 * u + qi;
-    const uint16_t* qp = qr + ((size_t)(r < m ? r : 0) * 8 + hq) * 256 + 8 * g;
+  for (int u = 0; u < 2; ++u)
 #pragma unroll
-    for (int s2 = 0; s2 < 8; ++s2) {
-      u32x4 v = *reinterpret_cast<const u32x4*>(qp + 32 * s2);
-      if (r >= m) v = u32x4{0u, 0u, 0u, 0u};
-      qf[u][s2] = __builtin_bit_cast(bf16x8, v);
-    }
-  }
+    for (int hd = 0; hd < 2; ++hd)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        qv[u][hd][j] = *reinterpret_cast<const u32x4*>(
+            qr + ((size_t)min(t0 + 16 * u + 4 * j + g, m - 1) * 8 + hq) * 256 + 128 * hd + 8 * qi);
   // DMA of one block of 32 keys: wave w moves rows 4w .. 4w+3 of K and V,
   // one row per instruction, lane L < 32 the row's 16-byte chunk L
   // Buffer resources over this KV head's rows of both caches: the row's byte
@@ -1344,6 +1348,36 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
   for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) ot[dt][r] = 0.0f;
+  // cleared here, while the loads are on their way
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt) asm volatile("" : "+v"(ot[dt]));
+  __builtin_amdgcn_sched_barrier(0);
+  // Q fragments: B operand of k-step s for query group u holds Q[16u + q][32s + 8g .. +7],
+  // through the wave's own part of the last stage, which the loop fills only
+  // after its first barrier (a group without queries repeats the other)
+  bf16x8 qf[2][8];
+  {
+    uint16_t* const ql = &kv[kFaStages - 1][wave * (16 * kFaQRow)];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int hd = 0; hd < 2; ++hd) {
+        if (u == 1 && t0 + 16 >= m) {
+#pragma unroll
+          for (int s2 = 0; s2 < 4; ++s2) qf[u][4 * hd + s2] = qf[0][4 * hd + s2];
+          continue;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4*>(ql + (4 * j + g) * kFaQRow + 8 * qi) = qv[u][hd][j];
+#pragma unroll
+        for (int s2 = 0; s2 < 4; ++s2)
+          qf[u][4 * hd + s2] = *reinterpret_cast<const bf16x8*>(ql + qi * kFaQRow + 32 * s2 + 8 * g);
+      }
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int s2 = 0; s2 < 8; ++s2) asm volatile("" : "+v"(qf[u][s2]));
   // The running reference starts below every score but finite: a row may have
   // no key in this wave's half of its blocks (or none before them), and
   // -inf - -inf would be NaN.
@@ -1355,6 +1389,7 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
   // keys 8(g / 2) .. of the wave's 16
   const uint32_t v_lane =
       (uint32_t)(2 * (32 * kFaKs + (16 * kh + 8 * (g >> 1) + (qi >> 2)) * kFaVs + 16 * (g & 1) + 4 * (qi & 3)));
+  int any_sums = 0;
   for (int kb = 0;; ++kb) {
     // blocks issued after kb and still in flight: min(kFaStages - 2, nkb-1-kb),
     // 8 DMA instructions each per wave
@@ -1438,13 +1473,15 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
     const float mrun_old = mrun;
     mrun = mnew;
     // factor is exactly 1 where the reference did not move: the rescale is
-    // skipped unless some lane's reference moved
-    if (__any(mnew > mrun_old)) {
+    // skipped unless some lane's reference moved and the sums are not still 0
+    if (any_sums && __any(mnew > mrun_old)) {
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) ot[dt][r] *= factor;
     }
+    any_sums = 1;
+    asm volatile("" : "+s"(any_sums));  // opaque: the first block is not peeled off the loop
     // O^T += V^T . P^T: one 16-key step per 32-dim tile
     const u32x4 pb = u32x4{pack2(pv[0], pv[1]), pack2(pv[2], pv[3]), pack2(pv[4], pv[5]), pack2(pv[6], pv[7])};
     const bf16x8 pf = __builtin_bit_cast(bf16x8, pb);
@@ -1460,40 +1497,83 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
         ot[4 * d4 + i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[i]), pf, ot[4 * d4 + i], 0, 0, 0);
     }
   }
-  // The upper half's wave leaves its state in the staging memory and raises its
-  // flag; the lower half's waits for it (the other wave runs on this CU and
-  // waits for nothing, so the wait ends) and writes the result.
-  float* merge = reinterpret_cast<float*>(&kv[0][0]) + (wave & 3) * (32 * 256 + 128);
+  // The two waves of a head each finish half of the dims, in their first four
+  // tiles: a wave leaves the sums of the other four and its softmax state in the
+  // staging memory, raises its flag and waits for the other's (both run on this
+  // CU and raise before they wait, so the wait ends). Key 0 is in the lower
+  // half, so the larger reference is a score's and the sum is not 0; an upper
+  // half without keys has weight 0. This and Q are the fixed cost of a tile,
+  // which shows where there are few keys (kernel us at position 0 for 8, 32,
+  // 128, 400 and 1000 queries: 16 queries and all keys to a wave 7.1, 10.5,
+  // 14.5, 23.5, 44.4; halves with Q straight into the fragments and one wave
+  // finishing all dims 9.5, 13.6, 17.2, 25.0, 43.4; this 8.3, 10.0, 13.4, 21.2,
+  // 39.6; at position 28672 849, 857, 859, 868, 891 against 967 .. 1010).
   if (kh) {
+    asm volatile("s_nop 15\n\ts_nop 15");  // past the last products' latency, which the compiler does not see here
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt)
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float lo = ot[dt][r], hi = ot[4 + dt][r];
+        asm volatile("v_swap_b32 %0, %1" : "+v"(lo), "+v"(hi));
+        ot[dt][r] = lo;
+        ot[4 + dt][r] = hi;
+      }
+  }
+  float* const mine = reinterpret_cast<float*>(&kv[0][0]) + wave * kFaMerge;
+  const float* const theirs = reinterpret_cast<const float*>(&kv[0][0]) + (wave ^ 4) * kFaMerge;
+  if (qvalid) {
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        *reinterpret_cast<float4*>(merge + ((4 * dt + r) * 64 + lane) * 4) =
-            make_float4(ot[dt][4 * r], ot[dt][4 * r + 1], ot[dt][4 * r + 2], ot[dt][4 * r + 3]);
-    merge[32 * 256 + lane] = mrun;
-    merge[32 * 256 + 64 + lane] = lrun;
-    __hip_atomic_store(&merged[wave & 3], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-    return;
+        *reinterpret_cast<float4*>(mine + ((4 * dt + r) * 64 + lane) * 4) =
+            make_float4(ot[4 + dt][4 * r], ot[4 + dt][4 * r + 1], ot[4 + dt][4 * r + 2], ot[4 + dt][4 * r + 3]);
+    mine[64 * 64 + lane] = mrun;
+    mine[64 * 65 + lane] = lrun;
   }
-  while (__hip_atomic_load(&merged[wave & 3], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
+  __hip_atomic_store(&merged[wave], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  while (__hip_atomic_load(&merged[wave ^ 4], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
     __builtin_amdgcn_s_sleep(1);
-  if (!qvalid) return;
-  // Key 0 is in the lower half, so mrun is a score's and the sum is not 0; an
-  // upper half without keys has weight 0.
-  const float m1 = merge[32 * 256 + lane], l1 = merge[32 * 256 + 64 + lane];
-  const float mx = fmaxf(mrun, m1), f0 = __builtin_amdgcn_exp2f(mrun - mx), f1 = __builtin_amdgcn_exp2f(m1 - mx);
-  const float inv = 1.0f / (lrun * f0 + l1 * f1), i0 = f0 * inv, i1 = f1 * inv;
-  uint16_t* op = o + ((size_t)qrow * 8 + hq) * 256 + 4 * (lane >> 5);
+  const float mo = theirs[64 * 64 + lane], lo = theirs[64 * 65 + lane];
+  const float m0 = kh ? mo : mrun, m1 = kh ? mrun : mo, l0 = kh ? lo : lrun, l1 = kh ? lrun : lo;
+  const float mx = fmaxf(m0, m1), f0 = __builtin_amdgcn_exp2f(m0 - mx), f1 = __builtin_amdgcn_exp2f(m1 - mx);
+  const float inv = 1.0f / (l0 * f0 + l1 * f1), i0 = f0 * inv, i1 = f1 * inv;
+  uint16_t* op = o + ((size_t)qrow * 8 + hq) * 256 + 128 * kh + 8 * (lane >> 5);
+  auto finish = [&](auto upper) {
+    constexpr bool U = decltype(upper)::value;  // own sums are the upper half's
 #pragma unroll
-  for (int dt = 0; dt < 8; ++dt)
+    for (int i = 0; i < 8; ++i) {
+      uint32_t w[4];  // dims 16 i + 4 (l / 32) .. + 3, and 8 further
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float4 u = *reinterpret_cast<const float4*>(merge + ((4 * dt + r) * 64 + lane) * 4);
-      *reinterpret_cast<uint2*>(op + 32 * dt + 8 * r) =
-          make_uint2(pack2(fmaf(ot[dt][4 * r], i0, u.x * i1), fmaf(ot[dt][4 * r + 1], i0, u.y * i1)),
-                     pack2(fmaf(ot[dt][4 * r + 2], i0, u.z * i1), fmaf(ot[dt][4 * r + 3], i0, u.w * i1)));
+      for (int r = 0; r < 2; ++r) {
+        const float4 u4 = *reinterpret_cast<const float4*>(theirs + ((2 * i + r) * 64 + lane) * 4);
+        const float u[4] = {u4.x, u4.y, u4.z, u4.w};
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float own = ot[i >> 1][4 * (2 * (i & 1) + r) + e];
+          v[e] = U ? fmaf(u[e], i0, own * i1) : fmaf(own, i0, u[e] * i1);
+        }
+        w[2 * r] = pack2(v[0], v[1]);
+        w[2 * r + 1] = pack2(v[2], v[3]);
+      }
+      // the halves of the wave exchange, so that a lane holds 8 dims in a row
+      const auto c01 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+      const auto c23 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+      if (qvalid) *reinterpret_cast<u32x4_a8*>(op + 16 * i) = u32x4{c01[0], c23[0], c01[1], c23[1]};
     }
+  };
+  // two bodies, kept apart: merged they select both operands of every product
+  if (kh) {
+    asm volatile("; upper half");
+    finish(std::true_type{});
+    asm volatile("; upper half done");
+  } else {
+    asm volatile("; lower half");
+    finish(std::false_type{});
+    asm volatile("; lower half done");
+  }
 }
 
 }  // namespace

@@ -44,3 +44,19 @@ def test_rows_do_not_depend_on_the_call():
     for lo, hi in ((0, 1), (1, 34), (17, 49), (90, 150)):
         print(f"case attn rows {lo}..{hi}", flush=True)
         assert np.array_equal(attend(query[lo:hi], kc, vc, pos0 + lo, hi - lo), full[lo:hi]), (lo, hi)
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 33])
+def test_output_rows_at_eight_byte_alignment(m):
+    """o four elements off 16-byte alignment: the same bits, nothing past the rows."""
+    print(f"case attn o alignment m={m}", flush=True)
+    r = rng(1500 + m)
+    query, kc, vc = (bf16(r.normal(0, 1, s)) for s in ((m, 2048), (2, m, 256), (2, m, 256)))
+    want = attend(query, kc, vc, 0, m)
+    d = [E.DeviceBuffer.from_numpy(a) for a in (query, kc, vc)]
+    do = E.DeviceBuffer.from_numpy(np.full(m * 2048 + 8, 0xA5A5, np.uint16))
+    E.check(E.lib().es_attn_prefill(d[0].ptr, d[1].ptr, d[2].ptr, 0, m, m, do.ptr + 8, None))
+    E.synchronize()
+    got = do.numpy(np.uint16)
+    assert np.array_equal(got[4:-4].reshape(m, 2048), want)
+    assert np.all(got[:4] == 0xA5A5) and np.all(got[-4:] == 0xA5A5)

@@ -161,6 +161,22 @@ def test_attention_prefill_barrier_waits(attn_asm):
     assert len(ops) == 8 and all(t.startswith("buffer_load_dwordx4") and t.endswith(" lds") for t in ops), ops
 
 
+def test_attention_prefill_queries_and_results_by_whole_lines(attn_asm):
+    """Before the loop a wave fetches its 32 queries of one head once, in 16
+    loads that each cover 256 bytes of four rows (two addresses a pair of
+    loads, 256 bytes apart, instead of 64 bytes of 16 rows); after it, each of
+    the two waves of a head writes half of the dims in 8 stores of 16 bytes a
+    lane (one body for each wave)."""
+    lines = [l.strip() for l in attn_asm]
+    bar = next(i for i, t in enumerate(lines) if t.startswith("s_barrier"))
+    loads = [t for t in lines[:bar] if t.startswith("global_load_")]
+    assert len(loads) == 16 and all(t.startswith("global_load_dwordx4") for t in loads), loads
+    assert sorted("offset:256" in t for t in loads) == [False] * 8 + [True] * 8
+    assert all("offset" not in t or t.endswith("offset:256") for t in loads)
+    stores = [t.split()[0] for t in lines[bar:] if t.startswith("global_store")]
+    assert stores == ["global_store_dwordx4"] * 16, stores
+
+
 def test_the_checker_follows_a_loop_back_edge():
     """A load issued at the end of a loop body and used at its top before a
     wait is flagged only when the back edge is walked."""

@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "es_kernels.hpp"
+#include "es_tiles.hpp"
 
 namespace es {
 namespace {
@@ -123,13 +124,12 @@ __global__ __launch_bounds__(256, 2) void k_q4_gemm(WideGemmArgs a, const uint16
   const int K = a.w[0].k, m = a.m, nk = K / kGemmBK;
   const int ncols = GATEUP ? a.w[0].n : a.nstart[a.nseg];
   int bx = blockIdx.x, by = blockIdx.y;
-  if (a.by_xcd) {  // block b goes to XCD b % 8: a row tile's blocks share an XCD and its L2's copy of X
-    const int nb = (ncols + 4 * kCols - 1) / (4 * kCols), i = bx >> 3;
-    by = (bx & 7) + 8 * (i / nb);
-    bx = i % nb;
+  if (a.by_xcd) {
+    const GemmTile tile = gemm_tile(blockIdx.x, (ncols + 4 * kCols - 1) / (4 * kCols), (m + kRows - 1) / kRows);
+    bx = tile.bx;
+    by = tile.by;
   }
   const int m0 = by * kRows;
-  if (m0 >= m) return;
 
   // Weight rows: lane l fetches chunk l % 8 of rows 8 i + l / 8 (i = 0..3) of
   // its wave's 32, and the scales (lanes 0..31) or biases (32..63) of row
@@ -1605,7 +1605,7 @@ static hipError_t launch_gemm_tiles(WideGemmArgs a, const uint16_t* residual, in
     a.vec = a.vec && ((uintptr_t)a.y[i] & 15) == 0 && (a.nstart[i + 1] - a.nstart[i]) % 8 == 0;
     lines = lines && (((uintptr_t)a.w[i].s | (uintptr_t)a.w[i].b) & 3) == 0;
   }
-  const dim3 grid = a.by_xcd ? dim3(8 * nb * ((mb + 7) / 8)) : dim3(nb, mb);
+  const dim3 grid = a.by_xcd ? dim3(gemm_grid(nb, mb)) : dim3(nb, mb);
   if (lines)
     hipLaunchKernelGGL((k_q4_gemm<MT, GATEUP, true>), grid, dim3(256), 0, s, a, residual);
   else

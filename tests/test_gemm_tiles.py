@@ -1,0 +1,51 @@
+"""The prefill GEMM's block-to-tile deal (csrc/es_tiles.hpp, plain C++, compiled
+here for the CPU): every tile is one block's, and the XCDs (block b runs on XCD
+b % 8) hold equal numbers of blocks, also where the row tiles are not a
+multiple of eight."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "enginesmith-qwen35-08b-long-decode-m5max-round005_amd", "csrc")
+PROGRAM = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "es_tiles.hpp"
+int main(int argc, char** argv) {  // column tiles, row tiles -> the grid's tiles in block order
+  const unsigned nb = atoi(argv[1]), mb = atoi(argv[2]);
+  for (unsigned b = 0; b < es::gemm_grid(nb, mb); ++b) {
+    const es::GemmTile t = es::gemm_tile(b, nb, mb);
+    printf("%d %d\n", t.bx, t.by);
+  }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    d = tmp_path_factory.mktemp("tiles")
+    (d / "tiles.cpp").write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, "-o", str(d / "tiles"), str(d / "tiles.cpp")], check=True)
+    return str(d / "tiles")
+
+
+# 56 and 65 column tiles: the MLP's gate/up and the stacked GDN input at 9, 10,
+# 17 and 32 tiles of 128 rows; odd and small ones
+@pytest.mark.parametrize("nb,mb", [(56, 9), (65, 9), (40, 10), (56, 17), (56, 32), (1, 8), (1, 9), (7, 15), (8, 8),
+                                   (13, 23), (28, 9)])
+def test_every_tile_once_and_the_xcds_equal(program, nb, mb):
+    out = subprocess.run([program, str(nb), str(mb)], check=True, capture_output=True, text=True).stdout
+    tiles = np.array(out.split(), int).reshape(-1, 2)
+    xcd = np.arange(len(tiles)) % 8
+    work = tiles[:, 1] < mb  # a block past the last row tile has none
+    tiles, xcd = tiles[work], xcd[work]
+    load = np.bincount(xcd, minlength=8)
+    assert load.max() - load.min() <= 1, load  # 9 x 56 dealt by whole row tiles: 112 and 56
+    assert len(tiles) == nb * mb
+    assert len(np.unique(tiles[:, 1] * nb + tiles[:, 0])) == nb * mb
+    assert tiles.min() == 0 and tiles[:, 0].max() == nb - 1 and tiles[:, 1].max() == mb - 1
+    whole = tiles[:, 1] < mb // 8 * 8  # the tiles dealt a row tile to an XCD
+    assert np.array_equal(tiles[whole, 1] % 8, xcd[whole])

@@ -78,14 +78,17 @@ def test_unaligned_outputs_and_scales(shift):
     assert np.array_equal(gemm(w2, x, n), want)
 
 
-@pytest.mark.parametrize("m,n", [(1, 8), (33, 24), (130, 1000), (300, 3584), (700, 3584)])
-def test_swiglu_tiles(m, n):
+# tiles of 32 rows; of 128; of 64 rows, in whole groups of steps and not; nine
+# and ten row tiles of 128, so a remainder after the eight dealt to the XCDs
+@pytest.mark.parametrize("m,n,k", [(1, 8, 320), (33, 24, 320), (130, 1000, 320), (300, 3584, 320), (700, 3584, 320),
+                                   (203, 3584, 320), (203, 3584, 1024), (1061, 3584, 320), (1061, 3584, 1024),
+                                   (1153, 1000, 1024)])
+def test_swiglu_tiles(m, n, k):
     """Gate and up interleaved in a wave's 32 weight rows: two GEMMs and
     es_swiglu_rows give the same bits, at each tile height and at widths that
     are not whole blocks of 64."""
-    print(f"case swiglu tiles m={m} n={n}", flush=True)
+    print(f"case swiglu tiles m={m} n={n} k={k}", flush=True)
     r = rng(8300 + m + n)
-    k = 320
     G, U = E.DeviceQ4(*random_q4(r, n, k)), E.DeviceQ4(*random_q4(r, n, k))
     x = bf16(r.normal(0, 1, (m, k)))
     dx = E.DeviceBuffer.from_numpy(x)

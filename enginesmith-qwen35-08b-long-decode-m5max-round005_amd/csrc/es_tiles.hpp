@@ -1,5 +1,5 @@
-// Which tile a GEMM block works on: plain C++, used by the kernels and by the
-// CPU test of the deal.
+// Which GEMM kernel a call takes and which tile a block works on: plain C++, used
+// by the kernels, their launchers and a CPU test.
 #pragma once
 
 namespace es {
@@ -24,6 +24,25 @@ constexpr GemmTile gemm_tile(unsigned b, unsigned nb, unsigned mb) {
   }
   const unsigned r = b - nb * whole;
   return {(int)(r % nb), (int)(whole + r / nb)};
+}
+
+// Whether a GEMM without residual goes to the kernel of 256 x 256 tiles: each
+// of its blocks has a CU to itself, so it is the faster one where the tiles fill
+// the 256 CUs in whole rounds, nearly (one round alone needs fewer: what it is
+// compared with is then two and a part), and where K is long enough for its
+// start and end, which nothing else on the CU covers, not to weigh. us, it and
+// the other kernel, rows x N x K:
+//   192 tiles, one round     3035 x 4096 x 3584 124 and 115   1499 x 8192 x 2048  73 and  66
+//   196 to 208, one round    3547 x 3584 x 3584 116 and 129   3291 x 4096 x 3584 119 and 128
+//   256, one round           4059 x 4096 x 3584 132 and 144   2011 x 8192 x 4096 144 and 161
+//   448 of 512               7131 x 4096 x 3584 248 and 238   3547 x 8192 x 2048 156 and 146
+//   480 of 512               5083 x 6144 x 3584 256 and 273   3803 x 8192 x 4096 277 and 301
+//   704 of 768              11227 x 4096 x 3584 375 and 373   2779 x 16384 x 2048 225 and 214
+//   728 of 768              13275 x 3584 x 3584 368 and 391
+//   K = 1024                 4096 x 6144 x 1024  81 and  67
+constexpr bool gemm_wide(int n, int k, int m) {
+  const long tiles = (long)((n + 255) / 256) * ((m + 255) / 256), rounds = (tiles + 255) / 256;
+  return k >= 2048 && k % 128 == 0 && tiles >= (rounds == 1 ? 196 : 240 * rounds);
 }
 
 }  // namespace es

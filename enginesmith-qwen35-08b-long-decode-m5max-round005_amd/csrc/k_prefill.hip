@@ -356,7 +356,7 @@ __global__ __launch_bounds__(256, 2) void k_q4_gemm(WideGemmArgs a, const uint16
     }
 }
 
-// ---- wide GEMM: 256 x 256 block tiles for a long K and many tiles (wide_ok) ----
+// ---- wide GEMM: 256 x 256 block tiles for a long K and many tiles (gemm_wide) ----
 //
 // k_q4_gemm_wide computes the same products as k_q4_gemm, bit for bit: the
 // same bf16 operands (weights dequantised as bf16(fma(scale, q, bias))) and,
@@ -1578,17 +1578,6 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
 
 }  // namespace
 
-// The wide kernel takes a GEMM without residual whose 256 x 256 tiles fill the
-// CUs (each block has one to itself) in rounds at least seven eighths full and
-// whose K is long enough for its start and end, which nothing else on the CU
-// covers, not to weigh (rows x N x K, wide against the other kernel, us:
-// 4096 x 4096 x 3584 121 and 134, 4096 x 8192 x 4096 266 and 302, but
-// 4096 x 6144 x 1024 81 and 67, 1000 x 8192 x 4096, half a round, 118 and 82).
-static bool wide_ok(int n, int k, int m) {
-  const long tiles = (long)((n + kWideN - 1) / kWideN) * ((m + kWideM - 1) / kWideM), rounds = (tiles + 255) / 256;
-  return k >= 2048 && k % (2 * kWideK) == 0 && tiles >= 224 * rounds;
-}
-
 static hipError_t launch_wide(const WideGemmArgs& a, hipStream_t s) {
   const dim3 grid((a.nstart[a.nseg] + kWideN - 1) / kWideN, (a.m + kWideM - 1) / kWideM);
   hipLaunchKernelGGL(k_q4_gemm_wide, grid, dim3(256), 0, s, a);
@@ -1620,7 +1609,7 @@ static hipError_t launch_gemm(const WideGemmArgs& a, const uint16_t* residual, h
   const int n = GATEUP ? a.w[0].n : a.nstart[a.nseg], cols = GATEUP ? 64 : 128;
   const int nb = (n + cols - 1) / cols;
   auto blocks = [&](int rows) { return (long)nb * ((a.m + rows - 1) / rows); };
-  if (!GATEUP && !residual && wide_ok(n, a.w[0].k, a.m)) return launch_wide(a, s);
+  if (!GATEUP && !residual && gemm_wide(n, a.w[0].k, a.m)) return launch_wide(a, s);
   if (blocks(32) <= 256) return launch_gemm_tiles<1, GATEUP>(a, residual, nb, s);
   if (blocks(64) <= 256) return launch_gemm_tiles<2, GATEUP>(a, residual, nb, s);
   return launch_gemm_tiles<4, GATEUP>(a, residual, nb, s);

@@ -1,7 +1,7 @@
 """The prefill GEMM's block-to-tile deal (csrc/es_tiles.hpp, plain C++, compiled
 here for the CPU): every tile is one block's, and the XCDs (block b runs on XCD
 b % 8) hold equal numbers of blocks, also where the row tiles are not a
-multiple of eight."""
+multiple of eight. And the rule for the kernel of 256 x 256 tiles."""
 import os
 import subprocess
 
@@ -22,14 +22,29 @@ int main(int argc, char** argv) {  // column tiles, row tiles -> the grid's tile
   }
 }
 """
+WIDE = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "es_tiles.hpp"
+int main(int argc, char** argv) { printf("%d", (int)es::gemm_wide(atoi(argv[1]), atoi(argv[2]), atoi(argv[3]))); }
+"""
+
+
+def compiled(tmp_path_factory, source):
+    d = tmp_path_factory.mktemp("tiles")
+    (d / "tiles.cpp").write_text(source)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, "-o", str(d / "tiles"), str(d / "tiles.cpp")], check=True)
+    return str(d / "tiles")
 
 
 @pytest.fixture(scope="module")
 def program(tmp_path_factory):
-    d = tmp_path_factory.mktemp("tiles")
-    (d / "tiles.cpp").write_text(PROGRAM)
-    subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, "-o", str(d / "tiles"), str(d / "tiles.cpp")], check=True)
-    return str(d / "tiles")
+    return compiled(tmp_path_factory, PROGRAM)
+
+
+@pytest.fixture(scope="module")
+def wide(tmp_path_factory):
+    return compiled(tmp_path_factory, WIDE)
 
 
 # 56 and 65 column tiles: the MLP's gate/up and the stacked GDN input at 9, 10,
@@ -49,3 +64,13 @@ def test_every_tile_once_and_the_xcds_equal(program, nb, mb):
     assert tiles.min() == 0 and tiles[:, 0].max() == nb - 1 and tiles[:, 1].max() == mb - 1
     whole = tiles[:, 1] < mb // 8 * 8  # the tiles dealt a row tile to an XCD
     assert np.array_equal(tiles[whole, 1] % 8, xcd[whole])
+
+
+# (N, K, rows) on both sides of the rule's lines, and which kernel measured faster
+@pytest.mark.parametrize("n,k,m,want", [
+    (4096, 3584, 3035, 0), (3584, 3584, 3547, 1), (4096, 3584, 3100, 1), (4096, 3584, 4096, 1), (8192, 4096, 1500, 0),
+    (4096, 3584, 7131, 0), (8192, 2048, 3547, 0), (6144, 3584, 5083, 1), (4096, 3584, 11227, 0), (3584, 3584, 13275, 1),
+    (6144, 1024, 4096, 0), (4096, 2112, 4096, 0)])
+def test_the_kernel_of_256_tiles_takes_what_it_is_faster_at(wide, n, k, m, want):
+    out = subprocess.run([wide, str(n), str(k), str(m)], check=True, capture_output=True, text=True).stdout
+    assert int(out) == want

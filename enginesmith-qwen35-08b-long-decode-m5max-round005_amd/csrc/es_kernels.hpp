@@ -219,7 +219,7 @@ hipError_t launch_q4_gemm_swiglu(const Q4& gate, const Q4& up, const uint16_t* x
                                  hipStream_t s);
 // Linears sharing one input, stacked along N (q|k|v, qkv|z|a|b): segment s
 // is Y_s[m, w[s].n] = bf16(X . W_s^T), bit for bit the separate linears.
-struct WideGemmArgs {
+struct GemmArgs {
   Q4 w[4];
   uint16_t* y[4];
   int nstart[5];  // first column of each segment; nstart[nseg] = total N

@@ -115,7 +115,7 @@ __device__ __forceinline__ float swiglu(float g, float u) {
 // a step for two bytes of scale. LINES: K is a multiple of 256 and the scales
 // allow four-byte accesses; otherwise the loads stay within the row one by one.
 template <int MT, bool GATEUP, bool LINES>
-__global__ __launch_bounds__(256, 2) void k_q4_gemm(WideGemmArgs a, const uint16_t* residual) {
+__global__ __launch_bounds__(256, 2) void k_q4_gemm(GemmArgs a, const uint16_t* residual) {
   constexpr int kRows = 32 * MT, D = kGemmAhead, kCols = GATEUP ? 16 : 32;  // output columns of a wave
   __shared__ __attribute__((aligned(16))) uint16_t xs[2][kRows * kGemmBK];
   __shared__ __attribute__((aligned(16))) uint16_t wl[4][32 * kGemmBK];
@@ -371,11 +371,10 @@ __global__ __launch_bounds__(256, 2) void k_q4_gemm(WideGemmArgs a, const uint16
 // fragment read touches cover all 64 banks once. The X DMA applies the same
 // permutation on the source side (lane l of an instruction fetches the chunk
 // that belongs in its slot).
-// Output columns may span up to four weight matrices stacked along N
-// (q|k|v, qkv|z|a|b), each written to its own [m][n_s] output.
 // A block holds a whole CU (128 KB of LDS, all registers), so nothing covers
 // its start and end: it is the faster kernel for a long K only.
 constexpr int kWideM = 256, kWideN = 256, kWideK = 64;
+static_assert(kWideM == 256 && kWideN == 256 && kWideK == 64, "gemm_wide counts these tiles, K in pairs of steps");
 
 // Fragment reads as inline assembly: the compiler treats an LDS read after a
 // DMA into LDS as dependent on it and would wait for every DMA in flight
@@ -434,28 +433,20 @@ __shared__ __attribute__((aligned(16))) uint16_t g_wide_x1[kWideM * kWideK];
 __shared__ __attribute__((aligned(16))) uint16_t g_wide_w0[kWideN * kWideK];
 __shared__ __attribute__((aligned(16))) uint16_t g_wide_w1[kWideN * kWideK];
 
-__global__ __launch_bounds__(256, 1) void k_q4_gemm_wide(WideGemmArgs a) {
+__global__ __launch_bounds__(256, 1) void k_q4_gemm_wide(Q4 w, const uint16_t* x, int m, uint16_t* y) {
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int K = a.w[0].k, m = a.m;
+  const int K = w.k;
   const int m0 = blockIdx.y * kWideM;
   const int nk = K / kWideK;
 
-  // this thread's weight row: segment, row within it, validity
+  // this thread's weight row
   const int n_row = blockIdx.x * kWideN + t;
-  int seg = 0;
-#pragma unroll
-  for (int sg = 1; sg < 4; ++sg)
-    if (sg < a.nseg && n_row >= a.nstart[sg]) seg = sg;
-  const int wrow = n_row - a.nstart[seg];
-  const bool wok = n_row < a.nstart[a.nseg];
-  const uint32_t* wcodes = seg == 0 ? a.w[0].w : seg == 1 ? a.w[1].w : seg == 2 ? a.w[2].w : a.w[3].w;
-  const uint16_t* wsc = seg == 0 ? a.w[0].s : seg == 1 ? a.w[1].s : seg == 2 ? a.w[2].s : a.w[3].s;
-  const uint16_t* wbi = seg == 0 ? a.w[0].b : seg == 1 ? a.w[1].b : seg == 2 ? a.w[2].b : a.w[3].b;
-  const int r_ok = wok ? wrow : 0;
-  const u32x4* cptr = reinterpret_cast<const u32x4*>(wcodes + (size_t)r_ok * (K >> 3));
-  const uint16_t* sptr = wsc + (size_t)r_ok * (K >> 6);
-  const uint16_t* bptr = wbi + (size_t)r_ok * (K >> 6);
+  const bool wok = n_row < w.n;
+  const int r_ok = wok ? n_row : 0;
+  const u32x4* cptr = reinterpret_cast<const u32x4*>(w.w + (size_t)r_ok * (K >> 3));
+  const uint16_t* sptr = w.s + (size_t)r_ok * (K >> 6);
+  const uint16_t* bptr = w.b + (size_t)r_ok * (K >> 6);
 
   // X DMA: instruction i of this wave fills LDS rows 8(8w+i) .. +7, lane l
   // the slot l & 7 of row l >> 3
@@ -466,7 +457,7 @@ __global__ __launch_bounds__(256, 1) void k_q4_gemm_wide(WideGemmArgs a) {
       const int r = (wave * 8 + i) * 8 + xr_lane;
       const int c = xslot ^ ((r >> 1) & 7);
       const int gr = min(m0 + r, m - 1);
-      const uint16_t* g = a.x + (size_t)gr * K + kb * kWideK + c * 8;
+      const uint16_t* g = x + (size_t)gr * K + kb * kWideK + c * 8;
       __builtin_amdgcn_global_load_lds(g, (lds_ptr_t)&xt[(wave * 8 + i) * 512], 16, 0, 0);
     }
   };
@@ -563,19 +554,13 @@ __global__ __launch_bounds__(256, 1) void k_q4_gemm_wide(WideGemmArgs a) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int n = blockIdx.x * kWideN + wn + 32 * j + fr;
-    if (n >= a.nstart[a.nseg]) continue;
-    int sg = 0;
-#pragma unroll
-    for (int q = 1; q < 4; ++q)
-      if (q < a.nseg && n >= a.nstart[q]) sg = q;
-    uint16_t* y = sg == 0 ? a.y[0] : sg == 1 ? a.y[1] : sg == 2 ? a.y[2] : a.y[3];
-    const int ld = a.nstart[sg + 1] - a.nstart[sg], col = n - a.nstart[sg];
+    if (n >= w.n) continue;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * fh + (r & 3);
-        if (row < m) y[(size_t)row * ld + col] = (uint16_t)f2bf(acc[i][j][r]);
+        if (row < m) y[(size_t)row * w.n + n] = (uint16_t)f2bf(acc[i][j][r]);
       }
   }
 }
@@ -1578,14 +1563,8 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
 
 }  // namespace
 
-static hipError_t launch_wide(const WideGemmArgs& a, hipStream_t s) {
-  const dim3 grid((a.nstart[a.nseg] + kWideN - 1) / kWideN, (a.m + kWideM - 1) / kWideM);
-  hipLaunchKernelGGL(k_q4_gemm_wide, grid, dim3(256), 0, s, a);
-  return hipGetLastError();
-}
-
 template <int MT, bool GATEUP>
-static hipError_t launch_gemm_tiles(WideGemmArgs a, const uint16_t* residual, int nb, hipStream_t s) {
+static hipError_t launch_gemm_tiles(GemmArgs a, const uint16_t* residual, int nb, hipStream_t s) {
   const int mb = (a.m + 32 * MT - 1) / (32 * MT);
   a.by_xcd = mb >= 8;  // fewer row tiles than XCDs: blocks in column order reach them all
   a.vec = ((uintptr_t)residual & 15) == 0;
@@ -1605,11 +1584,10 @@ static hipError_t launch_gemm_tiles(WideGemmArgs a, const uint16_t* residual, in
 // chip has CUs to spare and the time is one block's serial walk over K, which
 // a taller tile lengthens; past it the tallest tile dequantises least.
 template <bool GATEUP>
-static hipError_t launch_gemm(const WideGemmArgs& a, const uint16_t* residual, hipStream_t s) {
+static hipError_t launch_gemm(const GemmArgs& a, const uint16_t* residual, hipStream_t s) {
   const int n = GATEUP ? a.w[0].n : a.nstart[a.nseg], cols = GATEUP ? 64 : 128;
   const int nb = (n + cols - 1) / cols;
   auto blocks = [&](int rows) { return (long)nb * ((a.m + rows - 1) / rows); };
-  if (!GATEUP && !residual && gemm_wide(n, a.w[0].k, a.m)) return launch_wide(a, s);
   if (blocks(32) <= 256) return launch_gemm_tiles<1, GATEUP>(a, residual, nb, s);
   if (blocks(64) <= 256) return launch_gemm_tiles<2, GATEUP>(a, residual, nb, s);
   return launch_gemm_tiles<4, GATEUP>(a, residual, nb, s);
@@ -1618,7 +1596,7 @@ static hipError_t launch_gemm(const WideGemmArgs& a, const uint16_t* residual, h
 hipError_t launch_q4_gemm_stacked(const Q4* w, uint16_t* const* y, int nseg, const uint16_t* x, int m,
                                   hipStream_t s) {
   if (!w || !y || nseg < 1 || nseg > 4 || !x || m < 1) return hipErrorInvalidValue;
-  WideGemmArgs a{};
+  GemmArgs a{};
   int n = 0;
   for (int i = 0; i < nseg; ++i) {
     if (!w[i].w || !w[i].s || !w[i].b || !y[i] || w[i].n < 1 || w[i].k != w[0].k || w[i].k < kGemmBK ||
@@ -1645,7 +1623,12 @@ hipError_t launch_q4_gemm(const Q4& w, const uint16_t* x, int m, const uint16_t*
                           hipStream_t s) {
   if (!w.w || !w.s || !w.b || w.n < 1 || w.k < kGemmBK || w.k % kGemmBK != 0 || !x || !y || m < 1)
     return hipErrorInvalidValue;
-  const WideGemmArgs a{{w, w, w, w}, {y, y, y, y}, {0, w.n, w.n, w.n, w.n}, 1, x, m};
+  if (!residual && gemm_wide(w.n, w.k, m)) {
+    const dim3 grid((w.n + kWideN - 1) / kWideN, (m + kWideM - 1) / kWideM);
+    hipLaunchKernelGGL(k_q4_gemm_wide, grid, dim3(256), 0, s, w, x, m, y);
+    return hipGetLastError();
+  }
+  const GemmArgs a{{w, w, w, w}, {y, y, y, y}, {0, w.n, w.n, w.n, w.n}, 1, x, m};
   return launch_gemm<false>(a, residual, s);
 }
 
@@ -1654,7 +1637,7 @@ hipError_t launch_q4_gemm_swiglu(const Q4& gate, const Q4& up, const uint16_t* x
   if (!gate.w || !gate.s || !gate.b || !up.w || !up.s || !up.b || gate.n != up.n || gate.k != up.k ||
       gate.n < 1 || gate.k < kGemmBK || gate.k % kGemmBK != 0 || !x || !act || m < 1)
     return hipErrorInvalidValue;
-  const WideGemmArgs a{{gate, up, gate, up}, {act, act, act, act}, {0, gate.n, 2 * gate.n, 2 * gate.n, 2 * gate.n}, 2, x, m};
+  const GemmArgs a{{gate, up, gate, up}, {act, act, act, act}, {0, gate.n, 2 * gate.n, 2 * gate.n, 2 * gate.n}, 2, x, m};
   return launch_gemm<true>(a, nullptr, s);
 }
 

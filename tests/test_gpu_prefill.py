@@ -12,7 +12,7 @@ from helpers import assert_bf16_close, bf16, f32, random_q4, rng
 
 pytestmark = pytest.mark.gpu
 
-# N >= 2048 (K a multiple of 128) takes the 256 x 256 tiles, the rest the 128 x 128 tiles
+# tiles of 32, 64 and 128 rows by the number of blocks; K from one step of 64 on
 GEMM_SHAPES = [(1, 16, 1024), (17, 1024, 1024), (128, 128, 64), (300, 6144, 1024), (257, 1024, 3584),
                (2048, 512, 1024), (64, 1000, 2048), (130, 16, 1024), (1, 2048, 1024), (513, 2304, 1024),
                (257, 2048, 3584), (600, 4096, 2048)]
@@ -60,11 +60,13 @@ def test_q4_gemm_residual_in_place(k):
     assert np.mean(got != want) <= 0.01
 
 
-@pytest.mark.parametrize("m,k", [(1, 1024), (300, 1024), (513, 3584)])
+# the last two fill 200 and 216 tiles of 256 x 256 and take that kernel, their
+# halves and the others (one height, or 64-row tiles against 32) do not
+@pytest.mark.parametrize("m,k", [(1, 1024), (300, 1024), (513, 3584), (6300, 3584), (6657, 2048)])
 def test_wide_gemm_equals_narrow_tiles(m, k):
-    """An N = 2048 GEMM (256 x 256 tiles) and its two 1024-row halves as
-    separate GEMMs (128 x 128 tiles) give the same bits: every output element
-    is the same chain of MFMAs over K in both."""
+    """An N = 2048 GEMM and its two 1024-row halves as separate GEMMs give the
+    same bits: every output element is the same chain of MFMAs over K in both.
+    Rows at the edges of the tiles agree with the oracle."""
     print(f"case wide vs narrow m={m} k={k}", flush=True)
     r = rng(7000 + m + k)
     n = 2048
@@ -83,6 +85,10 @@ def test_wide_gemm_equals_narrow_tiles(m, k):
     full = dy.numpy(np.uint16).reshape(m, n)
     for h in range(2):
         assert np.array_equal(full[:, h * 1024:(h + 1) * 1024], dh[h].numpy(np.uint16).reshape(m, 1024))
+    rows = sorted({i for i in (0, 1, 127, 128, 255, 256, 300, m // 2, m - 1) if i < m})
+    # fp32 order only, as in test_q4_gemm
+    assert_bf16_close(full[rows], O.q4_gemm(codes, scales, biases, np.ascontiguousarray(x[rows])), max_ulp=1,
+                      max_frac=0.01, what=f"gemm {m}x{n}x{k}")
 
 
 def test_q4_gemm_rejects_bad_arguments():

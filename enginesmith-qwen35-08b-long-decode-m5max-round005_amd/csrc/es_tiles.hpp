@@ -1,5 +1,5 @@
-// Which GEMM kernel a call takes and which tile a block works on: plain C++, used
-// by the kernels, their launchers and a CPU test.
+// Which kernel a linear takes and which tile a block works on: plain C++, used by
+// the kernels, their launchers and a CPU test.
 #pragma once
 
 namespace es {
@@ -43,6 +43,24 @@ constexpr GemmTile gemm_tile(unsigned b, unsigned nb, unsigned mb) {
 constexpr bool gemm_wide(int n, int k, int m) {
   const long tiles = (long)((n + 255) / 256) * ((m + 255) / 256), rounds = (tiles + 255) / 256;
   return k >= 2048 && k % 128 == 0 && tiles >= (rounds == 1 ? 196 : 240 * rounds);
+}
+
+// Whether the matvec of several token rows gives a wave four weight rows (per
+// half-wave where K = 1024, half_wave) instead of one (two): outputs = token rows
+// x weight rows. A wave unpacks and sums its slices of x once for its weight rows
+// (about 100 instructions a slice, more than a row's dot product over it), so
+// four pay once their waves fill the 1024 SIMDs. Whole waves: at one a SIMD, not
+// where a few SIMDs get a second, and again from one and a half. Half-waves,
+// whose small form already has four weight rows a wave: from two and a half. us
+// with the small form and with four, outputs:
+//   K = 2048  4096 4.0 and 3.8   5120  4.5 and  4.7    6144  4.9 and  4.7   8192  5.8 and 4.7
+//   K = 1536  4096 3.7 and 3.7   5120  4.2 and  4.6    6144  4.7 and  4.7   8192  5.4 and 4.7
+//   K = 3584  4096 4.2 and 3.8   5120  4.7 and  4.8    6144  5.4 and  4.9  11264  8.3 and 6.4
+//   K = 1024 12288 3.2 and 3.5  18432  3.8 and  4.0   20480  3.8 and  4.0  21504  4.1 and 4.0   32768 4.9 and 4.5
+// Eight rows are slower again.
+constexpr bool qmv_four_rows(bool half_wave, long outputs) {
+  const long simds = 1024, waves = outputs / (half_wave ? 8 : 4);
+  return half_wave ? 8 * simds * 5 / 2 < outputs : waves == simds || 2 * waves >= 3 * simds;
 }
 
 }  // namespace es

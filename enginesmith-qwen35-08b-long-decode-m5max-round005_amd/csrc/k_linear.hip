@@ -16,6 +16,7 @@
 // Weight loads are issued at kernel entry, before the input and its RMSNorm,
 // so their latency overlaps that work.
 #include "es_kernels.hpp"
+#include "es_tiles.hpp"
 
 namespace es {
 namespace {
@@ -576,16 +577,8 @@ hipError_t launch_norm_gate_up_parts(const Q4& gate, const Q4& up, const uint16_
   return hipGetLastError();
 }
 
-// A wave unpacks and sums its slices of x once for its P weight rows (about
-// 100 instructions a slice, more than a row's dot product over it). One token
-// row has fewer waves than the chip has SIMDs, so P is small there; several
-// token rows take P = 4 once its waves fill the SIMDs (once for whole-wave
-// rows, twice for half-wave rows, whose P = 2 already holds four). us with the
-// small P and with 4, 11 token rows: 1024 x 3584 8.3 and 6.4, 3584 x 1024 5.65
-// and 5.2; 32 rows: 19.0 and 11.9, 12.2 and 10.0; at the line nothing either
-// way; P = 8 is slower again.
+// Weight rows a wave takes where qmv_four_rows says so.
 constexpr int kRowsP = 4;
-constexpr long kSimds = 1024;
 template <int P>
 static void launch_qmv_narrow_p(const Q4& w, const uint16_t* x, int rows, const uint16_t* residual, uint16_t* y,
                                 float* y_f32, hipStream_t s) {
@@ -610,12 +603,12 @@ hipError_t launch_qmv_rows(const Q4& w, const uint16_t* x, int rows, const uint1
   if (!q4_ok(w) || !x || !y || rows < 1 || rows > 65535 || (y_f32 && rows != 1))
     return hipErrorInvalidValue;
   if (w.k == kHidden) {
-    if (rows > 1 && (long)rows * w.n > 2 * kSimds * 2 * kRowsP)
+    if (rows > 1 && qmv_four_rows(true, (long)rows * w.n))
       launch_qmv_narrow_p<kRowsP>(w, x, rows, residual, y, y_f32, s);
     else
       launch_qmv_narrow_p<kNarrowP>(w, x, rows, residual, y, y_f32, s);
   } else if (w.k > kHidden && w.k <= 4096) {
-    if (rows > 1 && (long)rows * w.n >= kSimds * kRowsP)
+    if (rows > 1 && qmv_four_rows(false, (long)rows * w.n))
       launch_qmv_wide_p<kRowsP>(w, x, rows, residual, y, y_f32, s);
     else
       launch_qmv_wide_p<kWideP>(w, x, rows, residual, y, y_f32, s);

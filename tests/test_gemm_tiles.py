@@ -1,7 +1,8 @@
 """The prefill GEMM's block-to-tile deal (csrc/es_tiles.hpp, plain C++, compiled
 here for the CPU): every tile is one block's, and the XCDs (block b runs on XCD
 b % 8) hold equal numbers of blocks, also where the row tiles are not a
-multiple of eight. And the rule for the kernel of 256 x 256 tiles."""
+multiple of eight. And the rules for the kernel of 256 x 256 tiles and for four
+weight rows a wave in the matvec of several token rows."""
 import os
 import subprocess
 
@@ -27,6 +28,13 @@ WIDE = r"""
 #include <cstdlib>
 #include "es_tiles.hpp"
 int main(int argc, char** argv) { printf("%d", (int)es::gemm_wide(atoi(argv[1]), atoi(argv[2]), atoi(argv[3]))); }
+"""
+
+ROWS = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "es_tiles.hpp"
+int main(int argc, char** argv) { printf("%d", (int)es::qmv_four_rows(atoi(argv[1]) == 1024, atol(argv[2]))); }
 """
 
 
@@ -73,4 +81,14 @@ def test_every_tile_once_and_the_xcds_equal(program, nb, mb):
     (6144, 1024, 4096, 0), (4096, 2112, 4096, 0)])
 def test_the_kernel_of_256_tiles_takes_what_it_is_faster_at(wide, n, k, m, want):
     out = subprocess.run([wide, str(n), str(k), str(m)], check=True, capture_output=True, text=True).stdout
+    assert int(out) == want
+
+
+# (K, token rows x weight rows) on both sides of the lines, and which form measured faster
+@pytest.mark.parametrize("k,outputs,want", [
+    (2048, 3072, 0), (2048, 4096, 1), (1536, 5120, 0), (2048, 5120, 0), (2048, 6144, 1), (3584, 11264, 1),
+    (1024, 12288, 0), (1024, 18432, 0), (1024, 20480, 0), (1024, 21504, 1), (1024, 32768, 1)])
+def test_four_weight_rows_a_wave_where_they_are_faster(tmp_path_factory, k, outputs, want):
+    out = subprocess.run([compiled(tmp_path_factory, ROWS), str(k), str(outputs)], check=True, capture_output=True,
+                         text=True).stdout
     assert int(out) == want

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n,k,rows", [(1024, 3584, 3), (1024, 3584, 4), (1021, 2048, 5), (1026, 3584, 32),
                                       (3584, 1024, 4), (3584, 1024, 5), (3589, 1024, 7), (516, 1024, 33),
-                                      (1, 2048, 4100)])
+                                      (1, 2048, 4100), (1, 2048, 6145), (1021, 2048, 7), (516, 1024, 43)])
 def test_token_rows_by_four_weight_rows(n, k, rows):
     print(f"case matvec rows P n={n} k={k} rows={rows}", flush=True)
     r = rng(n + k + rows)

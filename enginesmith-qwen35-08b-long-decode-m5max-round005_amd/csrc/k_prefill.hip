@@ -889,6 +889,24 @@ __device__ __forceinline__ float recur_sum_and_readout(float& mem, const float (
         "v"(q[1]), "v"(q[2]), "v"(q[3]), "v"(q[4]), "v"(q[5]), "v"(q[6]), "v"(q[7]));
   return o;
 }
+// The updates S[i] = fma(k[i], delta, D[i]) (S holds D) with the same sum of the
+// readout o in the slots between them.
+__device__ __forceinline__ void recur_update_and_sum(float (&S)[8], const float (&k)[8], float delta, float& o) {
+  asm("v_fmac_f32 %0, %9, %17\n\t"
+      "v_fmac_f32 %1, %10, %17\n\t"
+      "v_add_f32_dpp %8, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32 %2, %11, %17\n\t"
+      "v_fmac_f32 %3, %12, %17\n\t"
+      "v_add_f32_dpp %8, %8, %8 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32 %4, %13, %17\n\t"
+      "v_fmac_f32 %5, %14, %17\n\t"
+      "v_add_f32_dpp %8, %8, %8 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32 %6, %15, %17\n\t"
+      "v_fmac_f32 %7, %16, %17\n\t"
+      "v_add_f32_dpp %8, %8, %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+      : "+v"(S[0]), "+v"(S[1]), "+v"(S[2]), "+v"(S[3]), "+v"(S[4]), "+v"(S[5]), "+v"(S[6]), "+v"(S[7]), "+v"(o)
+      : "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]), "v"(k[4]), "v"(k[5]), "v"(k[6]), "v"(k[7]), "v"(delta));
+}
 // The same sum alone.
 __device__ __forceinline__ float recur_sum(float v) {
   asm("s_nop 1\n\t"
@@ -1049,6 +1067,10 @@ __global__ __launch_bounds__(512, 1) void k_gdn_recur_rows(RecurIn in, int m, fl
     recur_read4(&tile[0].g[0], W.g[0]);
     recur_read4(&tile[0].v[rl][0], W.v[0]);
     recur_read4(&tile[0].beta[0], W.be[0]);
+    // The loop starts 44 bytes past a multiple of 256: where it falls in the
+    // instruction fetch counts 1% (4096 tokens, in turn: 377 us here, 380.5
+    // where it fell by itself).
+    asm volatile(".p2align 8\n\t.rept 9\n\ts_nop 0\n\t.endr");
     for (int i = 0; i < nfull; ++i) {
       const int nxt = cur == kRecurRing - 1 ? 0 : cur + 1;
       recur_walk_tile(tile[cur], tile[nxt], rl, l, W, i > 0 ? yrow + (size_t)(i - 1) * kRecurTile * 2048 : nullptr);
@@ -1061,25 +1083,48 @@ __global__ __launch_bounds__(512, 1) void k_gdn_recur_rows(RecurIn in, int m, fl
     W.p[15] = o;
     yrow[(size_t)((nfull - 1) * kRecurTile + recur_token(l)) * 2048] = (uint16_t)f2bf(recur_sum16(W.p, l));
   }
-  if (nfull < ntile) {  // the last m % 16 tokens
+  // The last m % 16 tokens, with operands in flight and readouts a token late as
+  // above (15 and 31 tokens: 5.2 and 7.1 us; with both sums alone after their
+  // products and each token's operands read when it starts, 5.6 and 7.7).
+  if (nfull < ntile) {
     const RecurTile& T = tile[cur];
-    for (int u = 0; u < m - nfull * kRecurTile; ++u) {
-      float k[8], q[8], mem = 0.0f, out = 0.0f;
-      recur_read8(T.k[u], l, k);
-      recur_read8(T.q[u], l, q);
+    const int rest = m - nfull * kRecurTile;  // < 16: the token after the last has a place in the tile
+    uint16_t* yt = yrow + (size_t)nfull * kRecurTile * 2048;
+    float g[2] = {T.g[0], 0.0f}, v[2] = {T.v[rl][0], 0.0f}, be[2] = {T.beta[0], 0.0f};
+    recur_read8(T.k[0], l, W.k[0]);
+    auto token = [&](int u, auto cc) {
+      constexpr int c = decltype(cc)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads issued a token ago
+      recur_read8(T.k[u + 1], l, W.k[c ^ 1]);
+      recur_read8(T.q[u], l, W.q[c]);
+      g[c ^ 1] = T.g[u + 1];
+      v[c ^ 1] = T.v[rl][u + 1];
+      be[c ^ 1] = T.beta[u + 1];
+      __builtin_amdgcn_sched_barrier(0);
+      float D[8], mem = 0.0f;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        W.S[i] = W.S[i] * T.g[u];
-        mem = fmaf(W.S[i], k[i], mem);
+        D[i] = W.S[i] * g[c];
+        mem = fmaf(D[i], W.k[c][i], mem);
       }
-      const float delta = (T.v[rl][u] - recur_sum(mem)) * T.beta[u];
+      float o = recur_sum_and_readout(mem, W.S, W.q[c ^ 1]);
+      const float delta = (v[c] - mem) * be[c];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        W.S[i] = fmaf(k[i], delta, W.S[i]);
-        out = fmaf(W.S[i], q[i], out);
+      for (int i = 0; i < 8; ++i) W.S[i] = D[i];
+      recur_update_and_sum(W.S, W.k[c], delta, o);
+      if (u > 0 && l == 0) yt[(size_t)(u - 1) * 2048] = (uint16_t)f2bf(o);
+      if (u == rest - 1) {
+        o = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o = fmaf(W.S[i], W.q[c][i], o);
+        o = recur_sum(o);
+        if (l == 0) yt[(size_t)u * 2048] = (uint16_t)f2bf(o);
       }
-      out = recur_sum(out);
-      if (l == 0) yrow[(size_t)(nfull * kRecurTile + u) * 2048] = (uint16_t)f2bf(out);
+    };
+    for (int u = 0; u < rest; u += 2) {
+      token(u, std::integral_constant<int, 0>{});
+      if (u + 1 < rest) token(u + 1, std::integral_constant<int, 1>{});
     }
     __syncthreads();  // barrier ntile
   }

@@ -177,6 +177,22 @@ def test_attention_prefill_queries_and_results_by_whole_lines(attn_asm):
     assert stores == ["global_store_dwordx4"] * 16, stores
 
 
+def test_recurrence_sums_run_between_other_products(tmp_path_factory):
+    """A DPP step that reads a register written by the instruction before it
+    waits two slots. In k_gdn_recur_rows two products stand there instead: in the
+    16 unrolled tokens of a whole tile before each of the memory sum's 4 steps,
+    and in the two bodies of a remainder token before those and before the 4 of
+    the readout of the token before."""
+    kernel_asm(tmp_path_factory, "k_gdn_recur_rows")  # compiles the file
+    lines = (tmp_path_factory.getbasetemp() / "k_prefill.s").read_text().splitlines()
+    start = next(i for i, l in enumerate(lines) if re.match(r"^_ZN2es12_GLOBAL__N_1\d+k_gdn_recur_rows\w*:", l))
+    ops = [l.split()[0] for l in lines[start:start + next(i for i, l in enumerate(lines[start:]) if ".section" in l)]
+           if re.match(r"\t[a-z]", l)]
+    filled = sum(a.startswith("v_fma") and b.startswith("v_fma") and c.startswith("v_add_f32_dpp")
+                 for a, b, c in zip(ops, ops[1:], ops[2:]))
+    assert filled >= 16 * 4 + 2 * (4 + 4), filled
+
+
 def test_the_checker_follows_a_loop_back_edge():
     """A load issued at the end of a loop body and used at its top before a
     wait is flagged only when the back edge is walked."""

@@ -1,5 +1,5 @@
-// Which kernel a linear takes and which tile a block works on: plain C++, used by
-// the kernels, their launchers and a CPU test.
+// Which form of a kernel a call takes and which tile a block works on: plain C++,
+// used by the kernels, their launchers and a CPU test.
 #pragma once
 
 namespace es {
@@ -62,5 +62,11 @@ constexpr bool qmv_four_rows(bool half_wave, long outputs) {
   const long simds = 1024, waves = outputs / (half_wave ? 8 : 4);
   return half_wave ? 8 * simds * 5 / 2 < outputs : waves == simds || 2 * waves >= 3 * simds;
 }
+
+// Whether the attention's output gate takes eight elements a thread (where the
+// pointers allow it) instead of one: below, fewer blocks finish later than more
+// do. us with one and with eight, rows: 64 1.9 and 2.1, 160 2.1 and 2.15, 203 2.2
+// and 2.15, 500 3.1 and 2.7, 4096 20.4 and 11.2.
+constexpr bool gate_eight(int rows) { return rows >= 192; }
 
 }  // namespace es

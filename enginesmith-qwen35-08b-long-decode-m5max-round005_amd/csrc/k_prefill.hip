@@ -1223,8 +1223,8 @@ __global__ __launch_bounds__(768) void k_attn_prep_rows(const uint16_t* qg, cons
 // Output gate rows (attn_gate, attention.metal:133-151): gated =
 // bf16(o * sigmoid_bf(gate)) with o the bf16 attention output and gate the
 // second half of each head's q_proj row.
-// V elements a thread: 8 where every pointer takes 16-byte accesses (4096 rows
-// 21 -> 11.6 us, 4.3 TB/s over 50 MB), else 1.
+// V elements a thread: 8 where gate_eight says so and every pointer takes 16-byte
+// accesses (4096 rows 20.4 -> 11.2 us, 4.5 TB/s over 50 MB), else 1.
 template <int V>
 __global__ __launch_bounds__(256) void k_attn_gate_rows(const uint16_t* o, const uint16_t* qg, int m,
                                                         uint16_t* gated) {
@@ -1792,7 +1792,7 @@ hipError_t launch_attn_prefill(const uint16_t* qr, const uint16_t* kcache, const
 hipError_t launch_attn_gate_rows(const uint16_t* o, const uint16_t* qg, int m, uint16_t* gated,
                                  hipStream_t s) {
   if (!o || !qg || !gated || m < 1 || m > (1 << 20) - 1) return hipErrorInvalidValue;  // m * 2048 < 2^31
-  if ((((uintptr_t)o | (uintptr_t)qg | (uintptr_t)gated) & 15) == 0)
+  if (gate_eight(m) && (((uintptr_t)o | (uintptr_t)qg | (uintptr_t)gated) & 15) == 0)
     hipLaunchKernelGGL(k_attn_gate_rows<8>, dim3(m), dim3(256), 0, s, o, qg, m, gated);
   else
     hipLaunchKernelGGL(k_attn_gate_rows<1>, dim3((m * 2048 + 255) / 256), dim3(256), 0, s, o, qg, m, gated);

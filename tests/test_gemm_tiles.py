@@ -1,8 +1,8 @@
 """The prefill GEMM's block-to-tile deal (csrc/es_tiles.hpp, plain C++, compiled
 here for the CPU): every tile is one block's, and the XCDs (block b runs on XCD
 b % 8) hold equal numbers of blocks, also where the row tiles are not a
-multiple of eight. And the rules for the kernel of 256 x 256 tiles and for four
-weight rows a wave in the matvec of several token rows."""
+multiple of eight. And the rules for the kernel of 256 x 256 tiles, for four weight
+rows a wave in the matvec of several token rows, and for the output gate."""
 import os
 import subprocess
 
@@ -35,6 +35,13 @@ ROWS = r"""
 #include <cstdlib>
 #include "es_tiles.hpp"
 int main(int argc, char** argv) { printf("%d", (int)es::qmv_four_rows(atoi(argv[1]) == 1024, atol(argv[2]))); }
+"""
+
+GATE = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "es_tiles.hpp"
+int main(int argc, char** argv) { printf("%d", (int)es::gate_eight(atoi(argv[1]))); }
 """
 
 
@@ -91,4 +98,10 @@ def test_the_kernel_of_256_tiles_takes_what_it_is_faster_at(wide, n, k, m, want)
 def test_four_weight_rows_a_wave_where_they_are_faster(tmp_path_factory, k, outputs, want):
     out = subprocess.run([compiled(tmp_path_factory, ROWS), str(k), str(outputs)], check=True, capture_output=True,
                          text=True).stdout
+    assert int(out) == want
+
+
+@pytest.mark.parametrize("rows,want", [(1, 0), (64, 0), (160, 0), (203, 1), (4096, 1)])
+def test_the_gate_takes_eight_elements_where_they_are_faster(tmp_path_factory, rows, want):
+    out = subprocess.run([compiled(tmp_path_factory, GATE), str(rows)], check=True, capture_output=True, text=True).stdout
     assert int(out) == want

@@ -29,12 +29,13 @@ def test_every_bf16_value():
     assert_bits_equal(np.where(nan, 0, got), np.where(nan, 0, want), what="silu")
 
 
+@pytest.mark.parametrize("m", [3, 191, 192, 193])
 @pytest.mark.parametrize("off", [0, 1])
-def test_gate_rows_aligned_and_not(off):
+def test_gate_rows_aligned_and_not(off, m):
     """Pointers `off` bf16 elements past 16-byte alignment take the element
-    form, aligned ones the 8-element form: the same bits, in place too."""
+    form, aligned ones the 8-element form from 192 rows: the same bits, in place
+    too."""
     r = np.random.default_rng(7)
-    m = 3
     o = O.f32_to_bf16(r.normal(0, 1, m * 2048).astype(np.float32))
     qp = O.f32_to_bf16(r.normal(0, 2, m * 4096).astype(np.float32))
     pad = np.zeros(off, np.uint16)

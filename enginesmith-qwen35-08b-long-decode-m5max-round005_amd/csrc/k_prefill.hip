@@ -1419,7 +1419,10 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
   // keys 8(g / 2) .. of the wave's 16
   const uint32_t v_lane =
       (uint32_t)(2 * (32 * kFaKs + (16 * kh + 8 * (g >> 1) + (qi >> 2)) * kFaVs + 16 * (g & 1) + 4 * (qi & 3)));
-  int any_sums = 0;
+  // The loop starts 44 bytes past a multiple of 256: where it falls in the
+  // instruction fetch counts up to 1% (4096 queries at 28672, in turn: 1019 us
+  // here, 1028 at 16 or 32 bytes).
+  asm volatile(".p2align 8\n\t.rept 7\n\ts_nop 0\n\t.endr");
   for (int kb = 0;; ++kb) {
     // blocks issued after kb and still in flight: min(kFaStages - 2, nkb-1-kb),
     // 8 DMA instructions each per wave
@@ -1503,15 +1506,13 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
     const float mrun_old = mrun;
     mrun = mnew;
     // factor is exactly 1 where the reference did not move: the rescale is
-    // skipped unless some lane's reference moved and the sums are not still 0
-    if (any_sums && __any(mnew > mrun_old)) {
+    // skipped unless some lane's reference moved
+    if (__any(mnew > mrun_old)) {
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) ot[dt][r] *= factor;
     }
-    any_sums = 1;
-    asm volatile("" : "+s"(any_sums));  // opaque: the first block is not peeled off the loop
     // O^T += V^T . P^T: one 16-key step per 32-dim tile
     const u32x4 pb = u32x4{pack2(pv[0], pv[1]), pack2(pv[2], pv[3]), pack2(pv[4], pv[5]), pack2(pv[6], pv[7])};
     const bf16x8 pf = __builtin_bit_cast(bf16x8, pb);
@@ -1534,10 +1535,10 @@ __global__ __launch_bounds__(512, 1) void k_attn_prefill(const uint16_t* qr, con
   // half, so the larger reference is a score's and the sum is not 0; an upper
   // half without keys has weight 0. This and Q are the fixed cost of a tile,
   // which shows where there are few keys (kernel us at position 0 for 8, 32,
-  // 128, 400 and 1000 queries: 16 queries and all keys to a wave 7.1, 10.5,
-  // 14.5, 23.5, 44.4; halves with Q straight into the fragments and one wave
-  // finishing all dims 9.5, 13.6, 17.2, 25.0, 43.4; this 8.3, 10.0, 13.4, 21.2,
-  // 39.6; at position 28672 849, 857, 859, 868, 891 against 967 .. 1010).
+  // 128, 400 and 1000 queries: 16 queries and all keys to a wave 7.0, 11.1,
+  // 14.5, 23.5, 44.5; halves with Q straight into the fragments and one wave
+  // finishing all dims 9.5, 14.3, 17.2, 25.0, 43.4; this 8.4, 10.4, 13.7, 21.5,
+  // 39.7; at position 28672 853, 854, 857, 875, 894 against 967 .. 1012).
   if (kh) {
     asm volatile("s_nop 15\n\ts_nop 15");  // past the last products' latency, which the compiler does not see here
 #pragma unroll

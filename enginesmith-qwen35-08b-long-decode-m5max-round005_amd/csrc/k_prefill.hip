@@ -66,11 +66,13 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t word, float sc, float bi) {
 // instructions of dequantisation (4 cycles each) that issue in their shadow:
 // MT = 4 balances them, smaller MT repeat the dequantisation for fewer rows.
 // Measured against a 128 x 128 kernel that staged both operands one step ahead
-// and stored its results one by one (us; the third and the last on 256 x 256
-// tiles before):
+// and stored its results one by one (us a launch in a graph's replay; the third
+// and the last on 256 x 256 tiles before; under the profiler, whose runs clock
+// lower, the present kernel's first, second, fourth and last take 26, 47, 89 and
+// 71):
 //   rows x N x K  203 x 1024 x 3584  4096 x 1024 x 3584  1000 x 4096 x 1024  4096 gate/up  4096 x 6144 x 1024
-//   before              55.7               82                  39                98              82
-//   now                 25.4               44                  16                81              67
+//   before              56                 81                  40               103              84
+//   now                 26                 45                  18                82              68
 constexpr int kGemmBK = 64, kGemmAhead = 4;
 
 // 16-byte chunk c of 64-column row r: chunk slot c ^ ((r >> 1) & 7), so the 16
@@ -779,8 +781,9 @@ __global__ __launch_bounds__(256) void k_gdn_prepare_hist(uint16_t* conv, const 
 // first two of its levels join lanes 8 and 4 apart, where DPP's bank mask
 // selects the token for free; every sum still joins the same key groups in the
 // same order ((0+1)+(2+3))+..., so the bits are the decode kernel's.
-// 4096 tokens: 374 us, 219 cycles a token (570 us with the readout after the
-// update and its own sum per token, and the walking waves staging the tiles).
+// 4096 tokens: 377 us in a graph's replay, 219 cycles a token (566 us with the
+// readout after the update and its own sum per token, and the walking waves
+// staging the tiles; under the profiler 388 us).
 // A copy without the LDS reads takes 340 us: the arithmetic's issue is what is
 // left.
 constexpr int kRecurTile = 16;
@@ -986,7 +989,7 @@ struct RecurWalk {
 // read here). While token u runs, token u + 1's k and token u's q (which the
 // readout uses during token u + 1) are in flight; the fences keep the reads
 // ahead of the arithmetic, and one wait per token covers them all (the
-// compiler's own placement waits three times a token: 389 against 374 us).
+// compiler's own placement waits three times a token: 4% slower).
 // The tile's own outputs but the last are complete at its end; yprev (when not
 // null) gets the 16 of the tile before.
 __device__ __forceinline__ void recur_walk_tile(const RecurTile& T, const RecurTile& next, int rl, int l, RecurWalk& W,
@@ -1253,8 +1256,8 @@ __global__ __launch_bounds__(256) void k_attn_gate_rows(const uint16_t* o, const
 // combined at the end. Every K and V fragment a wave reads from LDS so feeds
 // two products: with 16 queries and all 32 keys to a wave the LDS reads (256 KB
 // a key block, 2048 cycles at 128 bytes a cycle) took twice the products' 1024.
-// 4096 queries over 32768 keys: 1141 -> 1023 us in a graph's replay, 1.0
-// PFLOP/s (1237 us after under the profiler, whose runs clock lower).
+// 4096 queries over 32768 keys: 1141 -> 1020 us in a graph's replay, 1.0
+// PFLOP/s (1211 us after under the profiler, whose runs clock lower).
 // S^T = K . Q^T on 16x16x32 MFMAs (16 keys x two groups of 16 queries, K from
 // LDS, Q fragments in registers); a row swap per score leaves lane l with query
 // l % 32 and keys 8(l / 32) .. +7, so the online-softmax max and sum combine
